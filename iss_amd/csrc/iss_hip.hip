@@ -316,7 +316,7 @@ struct iss_ctx {
     int64_t dec_failed = 0;
     // smooth spectra
     DBuf<char> d_srec, d_sgrid;
-    DBuf<double> d_spart, d_sout;
+    DBuf<double> d_smilne, d_spart, d_sout;
     DBuf<int32_t> d_sspec;
     double spectra_ms = 0.;
 };
@@ -780,6 +780,12 @@ double mean_loss(iss_ctx* ctx, int nb) {
     return nv > 0. ? ls / nv : 0.;
 }
 
+template <int DF>
+void launch_spectra64(const SpectraArgs& a, dim3 grid, hipStream_t stream) {
+    if (a.positive_only) k_spectra64<DF, true><<<grid, 64, 0, stream>>>(a);
+    else k_spectra64<DF, false><<<grid, 64, 0, stream>>>(a);
+}
+
 template <typename R>
 int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species, int ns, const double* pT, int npT,
                 const double* phi, int nphi, const double* eta, const double* w, int ny, double* out) {
@@ -830,13 +836,20 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     HIPCHK(hipMemcpyAsync(ctx->d_sgrid.p, g.data(), sizeof(double) * g.size(), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(ctx->d_sspec.p, species, sizeof(int32_t) * ns, hipMemcpyHostToDevice, ctx->stream));
     const double* dg = reinterpret_cast<const double*>(ctx->d_sgrid.p);
-    // cell chunks: about 32 waves per CU over all (chunk, point-wave) pairs
+    // cell chunks: several rounds of resident waves over all (chunk,
+    // point-wave) pairs, so that the last, partly filled round is short
+    // (8 to 16 waves of these kernels fit a CU)
     const int64_t pw = ns * wps;
-    const int64_t target = static_cast<int64_t>(ctx->num_cu) * 32;
-    int64_t nch = std::max<int64_t>(1, std::min<int64_t>((target + pw - 1) / pw, (N + 7) / 8));
+    const bool milne = o->mode == 0 && sizeof(R) == sizeof(double);
+    const int64_t target = static_cast<int64_t>(ctx->num_cu) * 160;
+    int64_t nch = std::max<int64_t>(1, std::min<int64_t>((target + pw - 1) / pw, milne ? N : (N + 7) / 8));
     const int64_t cpc = (N + nch - 1) / nch;
     nch = (N + cpc - 1) / cpc;
-    HIPCHK(ctx->d_spart.ensure(nch * nout));
+    // the chunk sums are added in slices of chunks, then the slices
+    const int64_t oblk = (nout + 63) / 64;
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>((nch + 31) / 32, ctx->num_cu * 8 / oblk));
+    const int64_t per = (nch + want - 1) / want, nsl = (nch + per - 1) / per;
+    HIPCHK(ctx->d_spart.ensure((nch + nsl) * nout));
     HIPCHK(ctx->d_sout.ensure(nout));
     SpectraArgs a{};
     a.rec = rec;
@@ -859,9 +872,28 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     a.restrict_ratio = o->restrict_deltaf ? o->deltaf_max_ratio : 0.;
     a.waves_per_species = static_cast<int>(wps);
     a.partial = ctx->d_spart.p;
-    k_spectra<R><<<dim3(static_cast<unsigned>(nch), static_cast<unsigned>(pw)), 64, 0, ctx->stream>>>(a);
+    const dim3 grid(static_cast<unsigned>(nch), static_cast<unsigned>(pw));
+    if (milne) {
+        HIPCHK(ctx->d_smilne.ensure(static_cast<size_t>(kMilneRec) * N));
+        k_spectra_milne<<<(N + 63) / 64, 64, 0, ctx->stream>>>(rec, N, ctx->d_smilne.p);
+        a.milne = ctx->d_smilne.p;
+        // which terms the delta f has (k_spectra_rec leaves the others zero)
+        const bool poly_e = ctx->df.include_diffusion || (shear && ctx->neos == 1);
+        const bool const_e = bulk == BULK_RTA || bulk == BULK_CE;
+        if (poly_e) launch_spectra64<SDF_POLY_E>(a, grid, ctx->stream);
+        else if (const_e) launch_spectra64<SDF_CONST_E>(a, grid, ctx->stream);
+        else if (shear || bulk != BULK_NONE) launch_spectra64<SDF_POLY>(a, grid, ctx->stream);
+        else launch_spectra64<SDF_NONE>(a, grid, ctx->stream);
+    } else {
+        k_spectra<R><<<grid, 64, 0, ctx->stream>>>(a);
+    }
     HIPCHK(hipGetLastError());
-    k_spectra_reduce<<<(nout + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_spart.p, nch, nout, ctx->d_sout.p);
+    double* slices = ctx->d_spart.p + nch * nout;
+    k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), static_cast<unsigned>(nsl)), 256, 0, ctx->stream>>>(
+        ctx->d_spart.p, nch, per, nout, nsl > 1 ? slices : ctx->d_sout.p);
+    if (nsl > 1)
+        k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), 1), 256, 0, ctx->stream>>>(slices, nsl, nsl, nout,
+                                                                                        ctx->d_sout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
     HIPCHK(hipMemcpyAsync(out, ctx->d_sout.p, sizeof(double) * nout, hipMemcpyDeviceToHost, ctx->stream));
@@ -926,7 +958,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_ev_cell.release(); ctx->d_tr_spec.release(); ctx->d_ev_spec.release(); ctx->d_i32a.release();
     ctx->d_i32b.release(); ctx->d_f32a.release(); ctx->d_f32b.release(); ctx->d_f32c.release();
     ctx->d_cells_neg.release(); ctx->d_coef_neg.release(); ctx->d_srec.release(); ctx->d_sgrid.release();
-    ctx->d_spart.release(); ctx->d_sout.release(); ctx->d_sspec.release();
+    ctx->d_smilne.release(); ctx->d_spart.release(); ctx->d_sout.release(); ctx->d_sspec.release();
     ctx->d_surf_off.release(); ctx->d_bevents.release(); ctx->d_bround.release(); ctx->d_bevcount.release();
     ctx->d_bbase.release(); ctx->d_perms.release(); ctx->d_seg.release(); ctx->d_lam.release();
     for (auto& g : ctx->dgen) g->release();

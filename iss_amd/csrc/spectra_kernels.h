@@ -20,8 +20,9 @@
 // part of the integrand, k_spectra_rec) is read with wave-uniform (scalar)
 // loads, so the per-point work is pure VALU.  One wave evaluates 64 output
 // points over one contiguous chunk of cells; chunk sums go to
-// partial[chunk][species][point] in FP64 and k_spectra_reduce adds them in
-// chunk order (deterministic).
+// partial[chunk][species][point] in FP64 and k_spectra_reduce adds them in a
+// fixed order (deterministic).  FP64 spectra integrated over eta_s have a kernel
+// of their own (k_spectra64) on forms of the lab momentum.
 #pragma once
 
 #include "kernels.h"
@@ -134,6 +135,7 @@ struct SpectraArgs {
     double restrict_ratio;    // <= 0: no rescaling of delta f
     int waves_per_species;
     double* partial;          // [chunks][ns][npts]
+    const double* milne;      // [N][kMilneRec] (FP64, mode 0)
 };
 
 constexpr double kLog2e = 1.4426950408889634;
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(64) void k_spectra(SpectraArgs a) {
         c.qy = static_cast<R>(v[RS_QY]);
         c.qz = static_cast<R>(v[RS_QZ]);
         c.pq = static_cast<R>(v[RS_PQ]);
-        if (a.mode == 0) {
+        if (sizeof(R) == sizeof(float) && a.mode == 0) {  // (FP64 mode 0: k_spectra64)
             R mTr[kSpecPts], Pe[kSpecPts], Px[kSpecPts], Py[kSpecPts], Pz[kSpecPts], Pds[kSpecPts], X0[kSpecPts];
             R cell[kSpecPts];
 #pragma unroll
@@ -297,14 +299,276 @@ __global__ __launch_bounds__(64) void k_spectra(SpectraArgs a) {
     }
 }
 
-// out[i] = sum over chunks, in chunk order
-__global__ void k_spectra_reduce(const double* __restrict__ partial, int64_t nchunks, int64_t n,
-                                 double* __restrict__ out) {
+// ------------------------------------------------------ FP64, integrated over eta_s
+// The FP64 spectra of mode 0 are VALU-bound: N cells x n_eta nodes x points
+// evaluations of one integrand, so its FP64 instruction count is the time.
+// The kernel below evaluates the same sums with about 40 FP64 issue slots a
+// point where the rest-frame form (k_spectra) takes about 110:
+//   * Everything the integrand contracts is linear or quadratic in the lab
+//     momentum (mT cosh y, px, py, mT sinh y), and cosh, sinh of
+//     y = eta_cell + (y - eta_s)_k are linear in those of the node.  So per
+//     cell the record holds E, p.dsigma, q.l as linear forms and
+//     sa pi^{mu nu} p_mu p_nu + be2 E^2 (and sb pi^{mu nu} p_mu p_nu) as
+//     quadratic forms of (mT cosh y_k, mT sinh y_k, px, py); the whole
+//     delta f polynomial is 4 FMAs a point and needs neither E nor l.
+//   * The (cell, node) coefficients are formed once per wave, one node per
+//     lane, and read back from LDS as broadcasts (they cost about 20 FP64
+//     instructions per node and wave when every lane forms them).
+//   * 1 / E enters only where the delta f has it (Chapman-Enskog shear, the
+//     relaxation-time and Chapman-Enskog bulk, diffusion): DF.
+//   * exp2 is an 11-term polynomial on [-1/2, 1/2] (relative error 2e-17, 2e-16
+//     with its rounding) and an exponent shift, the reciprocal of the
+//     occupancy a hardware estimate with one third-order step (1 ulp).
+// Measured at 200,000 cells x 3 species x 720 points x 81 nodes: 98.8 ms
+// with k_spectra<double>, 40.5 ms with this kernel (8.6e11 points/s,
+// 31 of the 39 TFMA/s of the FP64 vector unit).
+constexpr int kMilneRec = 48;
+enum MilneSlot {
+    ML_IT = 0, ML_MB, ML_MS, ML_MQ,    // log2(e) / T and log2(e) mu / T
+    ML_E1, ML_E2, ML_U1, ML_U2,        // E = mT (E1 ch + E2 sh) - px U1 - py U2
+    ML_D1, ML_D2, ML_DX, ML_DY,        // p.dsigma, likewise (plus signs)
+    // quadratic form A = sa pi^{mu nu} p_mu p_nu + be2 E^2 (and B = sb pi pp):
+    // mT^2 (11 ch^2 + 12 ch sh + 22 sh^2) + mT px (1X ch + 2X sh) + mT py (1Y ch + 2Y sh)
+    // + XX px^2 + XY px py + YY py^2
+    ML_A,                              // 11, 12, 22, 1X, 2X, 1Y, 2Y, XX, XY, YY
+    ML_B = ML_A + 10,
+    ML_Q1 = ML_B + 10, ML_Q2, ML_QX, ML_QY,   // q.l / D_qmu, linear
+    ML_PQ, ML_BM2, ML_BE0, ML_BB, ML_BS, ML_BQ, ML_BM2E,
+    kMilneUsed
+};
+static_assert(kMilneUsed <= kMilneRec, "Milne spectra record");
+
+// the record of k_spectra_rec (rest frame) as forms of the lab momentum
+// relative to the cell's eta_s; one thread per cell
+__global__ void k_spectra_milne(const double* __restrict__ rec, int64_t N, double* __restrict__ out) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    if (i >= N) return;
+    const double* v = rec + i * kSpecRec;
+    double r[kMilneRec];
+    for (int k = 0; k < kMilneRec; k++) r[k] = 0.;
+    const double u0 = v[RS_U0], u1 = v[RS_U1], u2 = v[RS_U2], u3 = v[RS_U3], iu = v[RS_IU];
+    const double che = v[RS_CHE], she = v[RS_SHE];
+    r[ML_IT] = v[RS_IT] * kLog2e;
+    r[ML_MB] = v[RS_MB] * kLog2e;
+    r[ML_MS] = v[RS_MS] * kLog2e;
+    r[ML_MQ] = v[RS_MQ] * kLog2e;
+    r[ML_E1] = u0 * che - u3 * she;
+    r[ML_E2] = u0 * she - u3 * che;
+    r[ML_U1] = u1;
+    r[ML_U2] = u2;
+    // rest-frame momentum l = mT (ch b0 + sh b1) + px b2 + py b3
+    const double k1 = she * u3 * iu - che, k2 = che * u3 * iu - she, kx = u1 * iu, ky = u2 * iu;
+    const double b[4][3] = {{u1 * k1, u2 * k1, she + u3 * k1},
+                            {u1 * k2, u2 * k2, che + u3 * k2},
+                            {1. + u1 * kx, u2 * kx, u3 * kx},
+                            {u1 * ky, 1. + u2 * ky, u3 * ky}};
+    const double e[4] = {r[ML_E1], r[ML_E2], -u1, -u2};
+    // a temperature or chemical potential that is not a number makes every
+    // point so (the clamped exponent below would drop it)
+    const double poison = 0. * (v[RS_IT] + v[RS_MB] + v[RS_MS] + v[RS_MQ]);
+    for (int a = 0; a < 4; a++) {
+        r[ML_D1 + a] = e[a] * v[RS_D0] + b[a][0] * v[RS_D1] + b[a][1] * v[RS_D2] + b[a][2] * v[RS_D3] + poison;
+        r[ML_Q1 + a] = b[a][0] * v[RS_QX] + b[a][1] * v[RS_QY] + b[a][2] * v[RS_QZ];
+    }
+    const double xx = v[RS_XX], xy = 0.5 * v[RS_XY2], xz = 0.5 * v[RS_XZ2], yy = v[RS_YY], yz = 0.5 * v[RS_YZ2];
+    const double sa = v[RS_SA], sb = v[RS_SB], be2 = v[RS_BE2];
+    const int ia[10] = {0, 0, 1, 0, 1, 0, 1, 2, 2, 3}, ib[10] = {0, 1, 1, 2, 2, 3, 3, 2, 3, 3};
+#pragma unroll
+    for (int t = 0; t < 10; t++) {
+        const double* p = b[ia[t]];
+        const double* q = b[ib[t]];
+        const double w = p[0] * (xx * q[0] + xy * q[1] + xz * q[2]) + p[1] * (xy * q[0] + yy * q[1] + yz * q[2]) +
+                         p[2] * (xz * q[0] + yz * q[1] - (xx + yy) * q[2]);
+        const double f = ia[t] == ib[t] ? 1. : 2.;
+        r[ML_A + t] = f * (sa * w + be2 * e[ia[t]] * e[ib[t]]);
+        r[ML_B + t] = f * sb * w;
+    }
+    r[ML_PQ] = v[RS_PQ];
+    r[ML_BM2] = v[RS_BM2];
+    r[ML_BE0] = v[RS_BE0];
+    r[ML_BB] = v[RS_BB];
+    r[ML_BS] = v[RS_BS];
+    r[ML_BQ] = v[RS_BQ];
+    r[ML_BM2E] = v[RS_BM2E];
+    for (int k = 0; k < kMilneRec; k++) out[i * kMilneRec + k] = r[k];
+}
+
+// 2^x for |x| <= 1000: x = n + f, f in [-1/2, 1/2] (adding 1.5 2^52 rounds to
+// the nearest integer, whose low word is n), 2^f by a polynomial fitted at
+// the Chebyshev nodes of the interval
+__device__ __forceinline__ double exp2_poly(double x) {
+    const double magic = 6755399441055744.0;
+    const double t = x + magic;
+    const double f = x - (t - magic);
+    const int n = static_cast<int>(__builtin_bit_cast(uint64_t, t));
+    double p = 4.455446116749247e-10;
+    p = fma(p, f, 7.072590211349959e-09);
+    p = fma(p, f, 1.0178059415329878e-07);
+    p = fma(p, f, 1.3215442559248754e-06);
+    p = fma(p, f, 1.5252733836343741e-05);
+    p = fma(p, f, 0.00015403530441800403);
+    p = fma(p, f, 0.0013333558146411463);
+    p = fma(p, f, 0.009618129107606836);
+    p = fma(p, f, 0.05550410866482161);
+    p = fma(p, f, 0.24022650695910097);
+    p = fma(p, f, 0.6931471805599453);
+    p = fma(p, f, 1.0);
+    return __builtin_amdgcn_ldexp(p, n);
+}
+
+// 1 / d for finite normal d: the hardware estimate (about 2^-24) and one
+// third-order step, within 1 ulp
+__device__ __forceinline__ double rcp_step(double d) {
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fma(-d, r, 1.);
+    return fma(r, fma(e, e, e), r);
+}
+
+// delta f of the FP64 integrand: none, a polynomial, plus a constant over E,
+// plus a polynomial over E
+enum SpecDf { SDF_NONE = 0, SDF_POLY = 1, SDF_CONST_E = 2, SDF_POLY_E = 3 };
+
+// Grid (chunks, ns * waves_per_species), one wave per workgroup, kSpecPts
+// points per lane (points base + 64 q), nodes in groups of 64.
+template <int DF, bool POSITIVE>
+__global__ __launch_bounds__(64) void k_spectra64(SpectraArgs a) {
+    constexpr int NW = DF == SDF_POLY_E ? 12 : 8;   // doubles per node in LDS
+    __shared__ __align__(16) double s_node[64 * NW];
+    const int npts = a.npT * a.nphi;
+    const int si = blockIdx.y / a.waves_per_species;
+    const int lane = threadIdx.x;
+    const int base = (blockIdx.y % a.waves_per_species) * 64 * kSpecPts + lane;
+    const int s = a.species[si];
+    const double m = a.sp.mass[s], m2 = m * m;
+    const double B = a.sp.B[s], S = a.sp.S[s], Q = a.sp.Q[s], sg = a.sp.sign[s];
+    const double hi = a.restrict_ratio > 0. ? a.restrict_ratio : INFINITY;
+    double mT[kSpecPts], px[kSpecPts], py[kSpecPts], acc[kSpecPts];
+#pragma unroll
+    for (int q = 0; q < kSpecPts; q++) {
+        const int pt = min(base + 64 * q, npts - 1);
+        const double pT = a.pT[pt / a.nphi];
+        mT[q] = sqrt(pT * pT + m2);
+        px[q] = pT * a.cphi[pt % a.nphi];
+        py[q] = pT * a.sphi[pt % a.nphi];
+        acc[q] = 0.;
+    }
+    const int64_t l0 = static_cast<int64_t>(blockIdx.x) * a.cells_per_chunk;
+    const int64_t l1 = min<int64_t>(a.N, l0 + a.cells_per_chunk);
+    for (int64_t l = l0; l < l1; l++) {
+        const double* v = a.milne + l * kMilneRec;
+        const double it = v[ML_IT], mu = B * v[ML_MB] + S * v[ML_MS] + Q * v[ML_MQ];
+        const double be = v[ML_BE0] + B * v[ML_BB] + S * v[ML_BS] + Q * v[ML_BQ];
+        const double cm = v[ML_BM2] * m2, cme = v[ML_BM2E] * m2, pq = v[ML_PQ];
+        double X0[kSpecPts], Pds[kSpecPts], G0[kSpecPts], H0[kSpecPts], Pe[kSpecPts], cell[kSpecPts];
+#pragma unroll
+        for (int q = 0; q < kSpecPts; q++) {
+            Pe[q] = -(px[q] * v[ML_U1] + py[q] * v[ML_U2]);
+            X0[q] = fma(Pe[q], it, -mu);
+            Pds[q] = px[q] * v[ML_DX] + py[q] * v[ML_DY];
+            cell[q] = G0[q] = H0[q] = 0.;
+            if (DF != SDF_NONE)
+                G0[q] = px[q] * (px[q] * v[ML_A + 7] + py[q] * v[ML_A + 8]) + py[q] * py[q] * v[ML_A + 9] + cm +
+                        be * Pe[q];
+            if (DF == SDF_POLY_E) {
+                const double ql = px[q] * v[ML_QX] + py[q] * v[ML_QY];
+                G0[q] -= pq * ql;
+                H0[q] = px[q] * (px[q] * v[ML_B + 7] + py[q] * v[ML_B + 8]) + py[q] * py[q] * v[ML_B + 9] + cme +
+                        B * ql;
+            }
+        }
+        for (int k0 = 0; k0 < a.ny; k0 += 64) {
+            const int nk = min(64, a.ny - k0);
+            wave_lds_sync();
+            if (lane < nk) {
+                const double ch = a.ych[k0 + lane], sh = a.ysh[k0 + lane];
+                double* nd = s_node + lane * NW;
+                const double a0 = v[ML_E1] * ch + v[ML_E2] * sh;
+                nd[0] = DF >= SDF_CONST_E ? a0 : a0 * it;
+                nd[1] = v[ML_D1] * ch + v[ML_D2] * sh;
+                nd[2] = a.yw[k0 + lane];
+                if (DF != SDF_NONE) {
+                    nd[3] = ch * (v[ML_A + 0] * ch + v[ML_A + 1] * sh) + v[ML_A + 2] * sh * sh;
+                    nd[4] = v[ML_A + 3] * ch + v[ML_A + 4] * sh;
+                    nd[5] = v[ML_A + 5] * ch + v[ML_A + 6] * sh;
+                    nd[6] = be * a0;
+                }
+                if (DF == SDF_POLY_E) {
+                    const double ql = v[ML_Q1] * ch + v[ML_Q2] * sh;
+                    nd[6] -= pq * ql;
+                    nd[7] = ch * (v[ML_B + 0] * ch + v[ML_B + 1] * sh) + v[ML_B + 2] * sh * sh;
+                    nd[8] = v[ML_B + 3] * ch + v[ML_B + 4] * sh;
+                    nd[9] = v[ML_B + 5] * ch + v[ML_B + 6] * sh;
+                    nd[10] = B * ql;
+                }
+            }
+            wave_lds_sync();
+            for (int k = 0; k < nk; k++) {
+                double nd[NW];
+#pragma unroll
+                for (int t = 0; t < NW; t += 2) {
+                    const double2 w = *reinterpret_cast<const double2*>(s_node + k * NW + t);
+                    nd[t] = w.x;
+                    nd[t + 1] = w.y;
+                }
+#pragma unroll
+                for (int q = 0; q < kSpecPts; q++) {
+                    double E = 0., x;
+                    if (DF >= SDF_CONST_E) {
+                        E = fma(mT[q], nd[0], Pe[q]);
+                        x = fma(E, it, -mu);
+                    } else {
+                        x = fma(mT[q], nd[0], X0[q]);
+                    }
+                    // (2^+-1000: the occupancy is 0, or 1 / sg, to every digit)
+                    x = fmin(fmax(x, -1000.), 1000.);
+                    const double f0 = rcp_step(exp2_poly(x) + sg);
+                    double r = f0 * fma(mT[q], nd[1], Pds[q]);
+                    if (DF != SDF_NONE) {
+                        double G = fma(mT[q], fma(mT[q], nd[3], fma(px[q], nd[4], fma(py[q], nd[5], nd[6]))), G0[q]);
+                        if (DF == SDF_CONST_E) G = fma(rcp_step(E), cme, G);
+                        if (DF == SDF_POLY_E)
+                            G = fma(rcp_step(E),
+                                    fma(mT[q], fma(mT[q], nd[7], fma(px[q], nd[8], fma(py[q], nd[9], nd[10]))), H0[q]),
+                                    G);
+                        // |delta f| <= deltaf_max_ratio, as spectra_integrand
+                        const double df = fmin(fmax(fma(-sg, f0, 1.) * G, -hi), hi);
+                        r = fma(r, df, r);
+                    }
+                    if (POSITIVE && r < 0.) r = 0.;
+                    cell[q] = fma(nd[2], r, cell[q]);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kSpecPts; q++) acc[q] += cell[q];
+    }
+    const double pref = static_cast<double>(a.sp.g[s]) / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
+#pragma unroll
+    for (int q = 0; q < kSpecPts; q++) {
+        const int pt = base + 64 * q;
+        if (pt < npts) a.partial[(static_cast<int64_t>(blockIdx.x) * a.ns + si) * npts + pt] = acc[q] * pref;
+    }
+}
+
+// out[slice][i] = the sum over the slice's chunks (blockIdx.y, `per` chunks
+// each), in a fixed order: 64 consecutive outputs per workgroup, its four
+// waves take every fourth chunk.  Two launches (slices, then the slices'
+// sums) keep the whole chip loading where one thread per output would walk
+// all chunks alone (911 chunks x 2160 outputs: 221 us, now 2 x 9 us for 4546 chunks).
+__global__ __launch_bounds__(256) void k_spectra_reduce(const double* __restrict__ partial, int64_t nchunks,
+                                                        int64_t per, int64_t n, double* __restrict__ out) {
+    __shared__ double s_sum[4][64];
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + lane;
+    const int64_t t0 = blockIdx.y * per, t1 = min<int64_t>(nchunks, t0 + per);
     double s = 0.;
-    for (int64_t t = 0; t < nchunks; t++) s += partial[t * n + i];
-    out[i] = s;
+    if (i < n) {
+#pragma unroll 8
+        for (int64_t t = t0 + w; t < t1; t += 4) s += partial[t * n + i];
+    }
+    s_sum[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && i < n) out[blockIdx.y * n + i] = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
 }
 
 }  // namespace issdev
