@@ -28,8 +28,10 @@
 #include <memory>
 #include <cmath>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/iss_hip.h"
@@ -125,7 +127,7 @@ struct DBuf {
 // from device memory into pageable memory goes through the runtime's staging
 // buffer and costs tens of microseconds more than one into pinned memory.
 // Slots: PIN_OOB int, PIN_K int64, PIN_STATS 16 x u64, PIN_AUX 2 x int64, then
-// PIN_TOT [Ns] doubles.
+// PIN_MU int, PIN_TOT [Ns] doubles.
 struct PinBuf {
     void* p = nullptr;
     size_t cap = 0;
@@ -147,7 +149,7 @@ struct PinBuf {
     template <typename T>
     T* at(size_t off) { return reinterpret_cast<T*>(static_cast<char*>(p) + off); }
 };
-constexpr size_t PIN_OOB = 0, PIN_K = 8, PIN_STATS = 64, PIN_AUX = 192, PIN_TOT = 256;
+constexpr size_t PIN_OOB = 0, PIN_K = 8, PIN_STATS = 64, PIN_AUX = 192, PIN_MU = 208, PIN_TOT = 256;
 // device counters: [0..3] trials, |p| proposals, failed, out of table; [4..5]
 // learned fallback and envelope violations; [6..7] batch overflow flags; [8]
 // routed hadrons of batches; [9..12] the routed plain trials' [0..3]
@@ -186,6 +188,12 @@ struct DecayGen {
 
 }  // namespace
 
+// what tells one species' spectrum from another's, degeneracy aside
+struct SpeciesHost {
+    double mass;
+    int sign, B, S, Q;
+};
+
 struct iss_ctx {
     PinBuf h_pin;  // pinned read-back slots (PIN_*)
     int device = 0;
@@ -198,6 +206,7 @@ struct iss_ctx {
     // species
     int Ns = 0;
     std::vector<int> h_pid, h_charge, h_anti;
+    std::vector<SpeciesHost> h_sp;
     DBuf<int> d_anti;
     // local charge conservation: output positions' flags, partner offsets,
     // sources, partner set-up records, the second output list, new event offsets
@@ -233,6 +242,8 @@ struct iss_ctx {
     DBuf<uint32_t> d_u32;
     DBuf<int64_t> d_i64, d_scan;
     DBuf<double> d_eos;
+    DBuf<int> d_mu_used;
+    int mu_used = 0;  // which chemical potentials the surface has (MuUsed)
     // yields: LAYOUT_ROWS (k_yield_rows, the Poisson pass of one surface) or
     // LAYOUT_CDF (k_yield, FP64 species CDF rows: batches, multiplicity models)
     bool yields_valid = false;
@@ -465,23 +476,36 @@ DeltafDev deltaf_dev(iss_ctx* ctx) {
     return d;
 }
 
+// per-cell coefficients and words of the resident surface; returns when they
+// are ready
 int cell_prep(iss_ctx* ctx) {
+    HIPCHK(ctx->d_mu_used.ensure(1));
+    HIPCHK(ctx->h_pin.ensure(PIN_TOT));
+    int* h_mu = ctx->h_pin.at<int>(PIN_MU);
+    *h_mu = 0;
+    if (ctx->Nneg > 0 || ctx->Nc > 0) HIPCHK(hipMemsetAsync(ctx->d_mu_used.p, 0, sizeof(int), ctx->stream));
     if (ctx->Nneg > 0) {
         HIPCHK(ctx->d_coef_neg.ensure(kCoefRows * ctx->Nneg));
         k_cell_prep<<<(ctx->Nneg + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_cells_neg.p, ctx->Nneg, deltaf_dev(ctx),
-                                                                       ctx->d_coef_neg.p);
+                                                                       ctx->d_coef_neg.p, ctx->d_mu_used.p);
         HIPCHK(hipGetLastError());
     }
-    if (ctx->Nc == 0) return ISS_OK;
-    HIPCHK(ctx->d_coef.ensure(kCoefRows * ctx->Nc));
-    const int64_t nb = (ctx->Nc + 255) / 256;
-    k_cell_prep<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, deltaf_dev(ctx), ctx->d_coef.p);
-    HIPCHK(ctx->d_aux.ensure(static_cast<size_t>(kAuxFields) * ctx->Nc));
-    k_cell_aux<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_aux.p);
-    HIPCHK(hipGetLastError());
-    HIPCHK(ctx->d_ecell.ensure(2 * ctx->Nc));
-    k_emit_cells<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_ecell.p);
-    HIPCHK(hipGetLastError());
+    if (ctx->Nc > 0) {
+        HIPCHK(ctx->d_coef.ensure(kCoefRows * ctx->Nc));
+        const int64_t nb = (ctx->Nc + 255) / 256;
+        k_cell_prep<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, deltaf_dev(ctx), ctx->d_coef.p,
+                                                 ctx->d_mu_used.p);
+        HIPCHK(ctx->d_aux.ensure(static_cast<size_t>(kAuxFields) * ctx->Nc));
+        k_cell_aux<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_aux.p);
+        HIPCHK(hipGetLastError());
+        HIPCHK(ctx->d_ecell.ensure(2 * ctx->Nc));
+        k_emit_cells<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_ecell.p);
+        HIPCHK(hipGetLastError());
+    }
+    if (ctx->Nneg > 0 || ctx->Nc > 0)
+        HIPCHK(hipMemcpyAsync(h_mu, ctx->d_mu_used.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    ctx->mu_used = *h_mu;
     return ISS_OK;
 }
 
@@ -792,13 +816,13 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     const int64_t Nk = ctx->Nc, Nd = o->all_cells ? ctx->Nneg : 0, N = Nk + Nd;
     const int64_t npl = static_cast<int64_t>(npT) * nphi;
     const int64_t npts = npl * (o->mode == 1 ? ny : 1);
-    const int64_t nout = ns * npts;
+    const int64_t nall = ns * npts;
     if (npts > (int64_t{1} << 30)) return set_err(ctx, ISS_ERR_ARG, "spectra grid too large");
     const int64_t wps = (npts + 64 * kSpecPts - 1) / (64 * kSpecPts);
     if (ns * wps > 65535) return set_err(ctx, ISS_ERR_ARG, "spectra: species x grid points exceed one launch");
     ctx->spectra_ms = 0.;
     if (N == 0) {
-        std::fill(out, out + nout, 0.);
+        std::fill(out, out + nall, 0.);
         return ISS_OK;
     }
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
@@ -832,14 +856,36 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
         gp[oy + 2 * ny + k] = o->mode == 1 ? 1. : w[k];
     }
     HIPCHK(ctx->d_sgrid.ensure(sizeof(double) * g.size()));
-    HIPCHK(ctx->d_sspec.ensure(ns));
+    // Species of one mass, statistics and set of charges that matter have one
+    // integrand: it is evaluated once and scaled by each degeneracy (130 of
+    // the 321 UrQMD species where mu_S = mu_Q = 0; 314 with all potentials).
+    // A charge matters where its potential is not zero on every cell, or
+    // where it multiplies a bulk or diffusion term.
+    const bool c22 = bulk == BULK_22MOM;
+    const bool by_B = (ctx->mu_used & MU_B) || c22 || bulk == BULK_14MOM || ctx->df.include_diffusion;
+    const bool by_S = (ctx->mu_used & MU_S) || c22, by_Q = (ctx->mu_used & MU_Q) || c22;
+    std::vector<int32_t> spec(2 * static_cast<size_t>(ns));  // the species, then each one's evaluated species
+    std::vector<int32_t> reps;
+    std::map<std::tuple<double, int, int, int, int>, int32_t> seen;
+    for (int i = 0; i < ns; i++) {
+        const SpeciesHost& h = ctx->h_sp[species[i]];
+        const auto key = std::make_tuple(h.mass, h.sign, by_B ? h.B : 0, by_S ? h.S : 0, by_Q ? h.Q : 0);
+        const auto it = seen.emplace(key, static_cast<int32_t>(reps.size())).first;
+        if (it->second == static_cast<int32_t>(reps.size())) reps.push_back(species[i]);
+        spec[i] = species[i];
+        spec[ns + i] = it->second;
+    }
+    const int64_t nu = static_cast<int64_t>(reps.size()), nout = nu * npts;
+    spec.insert(spec.end(), reps.begin(), reps.end());
+    HIPCHK(ctx->d_sspec.ensure(spec.size()));
     HIPCHK(hipMemcpyAsync(ctx->d_sgrid.p, g.data(), sizeof(double) * g.size(), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(ctx->d_sspec.p, species, sizeof(int32_t) * ns, hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->d_sspec.p, spec.data(), sizeof(int32_t) * spec.size(), hipMemcpyHostToDevice,
+                          ctx->stream));
     const double* dg = reinterpret_cast<const double*>(ctx->d_sgrid.p);
     // cell chunks: several rounds of resident waves over all (chunk,
     // point-wave) pairs, so that the last, partly filled round is short
     // (8 to 16 waves of these kernels fit a CU)
-    const int64_t pw = ns * wps;
+    const int64_t pw = nu * wps;
     const bool milne = o->mode == 0 && sizeof(R) == sizeof(double);
     const int64_t target = static_cast<int64_t>(ctx->num_cu) * 160;
     int64_t nch = std::max<int64_t>(1, std::min<int64_t>((target + pw - 1) / pw, milne ? N : (N + 7) / 8));
@@ -849,15 +895,15 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     const int64_t oblk = (nout + 63) / 64;
     const int64_t want = std::max<int64_t>(1, std::min<int64_t>((nch + 31) / 32, ctx->num_cu * 8 / oblk));
     const int64_t per = (nch + want - 1) / want, nsl = (nch + per - 1) / per;
-    HIPCHK(ctx->d_spart.ensure((nch + nsl) * nout));
-    HIPCHK(ctx->d_sout.ensure(nout));
+    HIPCHK(ctx->d_spart.ensure((nch + nsl + 1) * nout));
+    HIPCHK(ctx->d_sout.ensure(nall));
     SpectraArgs a{};
     a.rec = rec;
     a.N = N;
     a.cells_per_chunk = cpc;
     a.sp = species_dev(ctx);
-    a.species = ctx->d_sspec.p;
-    a.ns = ns;
+    a.species = ctx->d_sspec.p + 2 * ns;
+    a.ns = static_cast<int>(nu);
     a.pT = dg;
     a.npT = npT;
     a.cphi = dg + npT;
@@ -888,15 +934,17 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
         k_spectra<R><<<grid, 64, 0, ctx->stream>>>(a);
     }
     HIPCHK(hipGetLastError());
-    double* slices = ctx->d_spart.p + nch * nout;
+    double* sums = ctx->d_spart.p + nch * nout;
+    double* slices = sums + nout;
     k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), static_cast<unsigned>(nsl)), 256, 0, ctx->stream>>>(
-        ctx->d_spart.p, nch, per, nout, nsl > 1 ? slices : ctx->d_sout.p);
+        ctx->d_spart.p, nch, per, nout, nsl > 1 ? slices : sums);
     if (nsl > 1)
-        k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), 1), 256, 0, ctx->stream>>>(slices, nsl, nsl, nout,
-                                                                                        ctx->d_sout.p);
+        k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), 1), 256, 0, ctx->stream>>>(slices, nsl, nsl, nout, sums);
+    k_spectra_spread<<<(nall + 255) / 256, 256, 0, ctx->stream>>>(sums, ctx->d_sspec.p, ctx->d_sspec.p + ns, a.sp.g,
+                                                                  npts, nall, ctx->d_sout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    HIPCHK(hipMemcpyAsync(out, ctx->d_sout.p, sizeof(double) * nout, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipMemcpyAsync(out, ctx->d_sout.p, sizeof(double) * nall, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
@@ -941,7 +989,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_mass.release(); ctx->d_spk.release(); ctx->d_ints.release(); ctx->d_k11.release(); ctx->d_neos.release();
     ctx->d_ktab.release(); ctx->d_ktabf.release(); ctx->d_ptab.release();
     ctx->d_cells.release(); ctx->d_tmp.release(); ctx->d_coef.release(); ctx->d_u32.release();
-    ctx->d_i64.release(); ctx->d_scan.release(); ctx->d_eos.release(); ctx->d_cdf.release();
+    ctx->d_i64.release(); ctx->d_mu_used.release(); ctx->d_scan.release(); ctx->d_eos.release(); ctx->d_cdf.release();
     ctx->d_ctot.release(); ctx->d_partial.release(); ctx->d_oob.release(); ctx->d_stot.release(); ctx->d_raw.release();
     ctx->d_counts.release(); ctx->d_evcount.release(); ctx->d_off.release(); ctx->d_evoff.release();
     ctx->d_tree0.release(); ctx->d_tree1.release(); ctx->d_out.release(); ctx->d_setup.release(); ctx->d_stats.release();
@@ -1061,6 +1109,9 @@ int iss_set_species(iss_ctx* ctx, const iss_species_desc* sp) {
         HIPCHK(hipMemcpy(ctx->d_rowsp.p, rs.data(), sizeof(RowSp) * rs.size(), hipMemcpyHostToDevice));
     }
     ctx->h_pid.assign(sp->pid, sp->pid + Ns);
+    ctx->h_sp.resize(Ns);
+    for (int i = 0; i < Ns; i++)
+        ctx->h_sp[i] = SpeciesHost{sp->mass[i], sp->sign[i], sp->baryon[i], sp->strange[i], sp->charge[i]};
     ctx->h_charge.assign(sp->charge, sp->charge + Ns);
     // antiparticle entries (local charge conservation)
     ctx->h_anti.assign(Ns, -1);
@@ -1136,10 +1187,7 @@ int iss_set_deltaf(iss_ctx* ctx, const iss_deltaf_desc* d) {
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->tables_ready = true;
     ctx->yields_valid = false;
-    rc = cell_prep(ctx);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return ISS_OK;
+    return cell_prep(ctx);
 }
 
 int iss_set_surface_lab(iss_ctx* ctx, int64_t n, const float* cells34, const iss_eos_desc* eos) {
@@ -1191,10 +1239,7 @@ int iss_set_surface_lab(iss_ctx* ctx, int64_t n, const float* cells34, const iss
     lab.release();
     ctx->Nc = nk;
     ctx->Nneg = n - nk;
-    rc = cell_prep(ctx);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return ISS_OK;
+    return cell_prep(ctx);
 }
 
 int iss_set_surface_lrf(iss_ctx* ctx, int64_t n, const float* cells28) {
@@ -1211,10 +1256,7 @@ int iss_set_surface_lrf(iss_ctx* ctx, int64_t n, const float* cells28) {
     k_aos_to_soa<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_tmp.p, n, ctx->d_cells.p);
     HIPCHK(hipGetLastError());
     ctx->Nc = n;
-    int rc = cell_prep(ctx);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return ISS_OK;
+    return cell_prep(ctx);
 }
 
 int64_t iss_num_cells(const iss_ctx* ctx) { return ctx ? ctx->Nc : -1; }

@@ -117,7 +117,7 @@ struct SpectraArgs {
     int64_t N;
     int64_t cells_per_chunk;
     SpeciesDev sp;
-    const int32_t* species;   // [ns] species indices
+    const int32_t* species;   // [ns] species indices, one of each set with equal integrands
     int ns;
     const double* pT;         // [npT]
     int npT;
@@ -290,12 +290,10 @@ __global__ __launch_bounds__(64) void k_spectra(SpectraArgs a) {
             }
         }
     }
-    const double g = static_cast<double>(a.sp.g[s]);
-    const double pref = g / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
 #pragma unroll
     for (int q = 0; q < kSpecPts; q++) {
         const int pt = base + 64 * q;
-        if (pt < npts) a.partial[(static_cast<int64_t>(blockIdx.x) * a.ns + si) * npts + pt] = acc[q] * pref;
+        if (pt < npts) a.partial[(static_cast<int64_t>(blockIdx.x) * a.ns + si) * npts + pt] = acc[q];
     }
 }
 
@@ -542,11 +540,10 @@ __global__ __launch_bounds__(64) void k_spectra64(SpectraArgs a) {
 #pragma unroll
         for (int q = 0; q < kSpecPts; q++) acc[q] += cell[q];
     }
-    const double pref = static_cast<double>(a.sp.g[s]) / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
 #pragma unroll
     for (int q = 0; q < kSpecPts; q++) {
         const int pt = base + 64 * q;
-        if (pt < npts) a.partial[(static_cast<int64_t>(blockIdx.x) * a.ns + si) * npts + pt] = acc[q] * pref;
+        if (pt < npts) a.partial[(static_cast<int64_t>(blockIdx.x) * a.ns + si) * npts + pt] = acc[q];
     }
 }
 
@@ -569,6 +566,18 @@ __global__ __launch_bounds__(256) void k_spectra_reduce(const double* __restrict
     s_sum[w][lane] = s;
     __syncthreads();
     if (w == 0 && i < n) out[blockIdx.y * n + i] = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
+}
+
+// out[s] = g_s / (2 pi hbar c)^3 times the sum of the species it shares its
+// integrand with (pick[s], an index into the evaluated species)
+__global__ void k_spectra_spread(const double* __restrict__ sum, const int32_t* __restrict__ species,
+                                 const int32_t* __restrict__ pick, const int* __restrict__ g, int64_t npts, int64_t n,
+                                 double* __restrict__ out) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int64_t s = i / npts;
+    const double pref = static_cast<double>(g[species[s]]) / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
+    out[i] = sum[pick[s] * npts + (i - s * npts)] * pref;
 }
 
 }  // namespace issdev

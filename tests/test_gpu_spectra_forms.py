@@ -94,3 +94,28 @@ def test_far_rapidities_and_positive_only():
     out = ctx.spectra(idx, pT, phi, eta, w, mode=0, precision=64, use_pos_dN_only=1)
     assert np.all(np.isfinite(out)) and np.all(out >= 0)
     ctx.close()
+
+
+@pytest.mark.parametrize("name", ["ideal", "rta", "osu14", "mom22", "diffusion"])
+@pytest.mark.parametrize("potentials", ["none", "B", "BQ", "S"])
+@pytest.mark.parametrize("precision", [32, 64])
+def test_species_evaluated_together_equal_species_alone(name, potentials, precision):
+    """One call for species that share masses and charges against one call
+    per species: the same sums up to the grouping of cells into chunks (FP64
+    sums of 60 cells: 1e-13)."""
+    c = _cells(60, 9)
+    c[:, 16] *= "B" in potentials
+    c[:, 17] *= "S" in potentials
+    c[-1, 18] = 0.02 if "Q" in potentials else 0.0   # (one cell alone has mu_Q)
+    c[:-1, 18] = 0.0
+    ctx = _context(name, c)
+    sp = tables.species_arrays(1)
+    idx = np.array([0, 1, 2, 3, 4, 5, 6, 0, 16, 17, 18, 19, 21, 22, 40, 41, 42, 43])
+    assert len(set(zip(sp["mass"][idx], sp["B"][idx]))) < idx.size
+    pT, phi, eta, w = np.linspace(0.1, 2.0, 4), np.linspace(0, 5.5, 6), np.linspace(-2, 2, 9), np.full(9, 0.5)
+    for mode in (0, 1):
+        together = ctx.spectra(idx, pT, phi, eta, w, mode=mode, precision=precision)
+        alone = np.stack([ctx.spectra([i], pT, phi, eta, w, mode=mode, precision=precision)[0] for i in idx])
+        scale = np.abs(alone).max(axis=-1, keepdims=True)
+        assert np.all(np.abs(together - alone) <= 1e-13 * scale)
+    ctx.close()
