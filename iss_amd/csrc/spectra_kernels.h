@@ -112,6 +112,23 @@ __global__ void k_spectra_rec(const float* __restrict__ cells, const double* __r
     for (int k = 0; k < kSpecRec; k++) rec[i * kSpecRec + k] = r[k];
 }
 
+// Which chemical potentials (over T) are not zero on some cell (NaN counts),
+// as bits in *used: one atomic per workgroup, so that few meet on the word.
+enum MuUsed { MU_B = 1, MU_S = 2, MU_Q = 4 };
+__global__ __launch_bounds__(256) void k_mu_used(const double* __restrict__ rec, int64_t N, int* __restrict__ used) {
+    int m = 0;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < N;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        const double* v = rec + i * kSpecRec;
+        m |= !(v[RS_MB] == 0.) ? MU_B : 0;
+        m |= !(v[RS_MS] == 0.) ? MU_S : 0;
+        m |= !(v[RS_MQ] == 0.) ? MU_Q : 0;
+    }
+    const int b = __syncthreads_or(m & MU_B), s = __syncthreads_or(m & MU_S), q = __syncthreads_or(m & MU_Q);
+    m = (b ? MU_B : 0) | (s ? MU_S : 0) | (q ? MU_Q : 0);
+    if (threadIdx.x == 0 && m) atomicOr(used, m);
+}
+
 struct SpectraArgs {
     const double* rec;        // [N][kSpecRec]
     int64_t N;

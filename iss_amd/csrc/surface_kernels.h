@@ -336,18 +336,10 @@ __global__ void k_expint_table(double* etab) {
 
 // Per-cell coefficients as the yield loop selects them (src/FSSW.cpp:597-637);
 // rows 6, 7: 1 / deltaf_qmu_coeff and n_B / (e + P) of the diffusion delta f.
-// mu_used collects which chemical potentials are not zero everywhere (bit 0
-// mu_B, 1 mu_S, 2 mu_Q): the spectra evaluate species that differ only in a
-// charge without a potential once.
-enum MuUsed { MU_B = 1, MU_S = 2, MU_Q = 4 };
 __global__ void k_cell_prep(const float* __restrict__ cells, int64_t Nc, DeltafDev d,
-                            double* __restrict__ coef, int* __restrict__ mu_used) {
+                            double* __restrict__ coef) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= Nc) return;
-    int used = !(cells[F_MUB * Nc + i] == 0.f) ? MU_B : 0;  // (NaN counts as used)
-    if (!(cells[F_MUS * Nc + i] == 0.f)) used |= MU_S;
-    if (!(cells[F_MUQ * Nc + i] == 0.f)) used |= MU_Q;
-    if (used & ~__hip_atomic_load(mu_used, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(mu_used, used);
     double c[6] = {0., 0., 0., 0., 0., 0.};
     const double T = cells[F_T * Nc + i], muB = cells[F_MUB * Nc + i];
     const double Ed = cells[F_E * Nc + i], nB = cells[F_NB * Nc + i];
