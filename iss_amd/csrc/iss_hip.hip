@@ -337,12 +337,14 @@ struct iss_ctx {
     int yield_precision = 0;
     int yield_layout = 0;
     int nlight = 0;  // leading species below 0.7 GeV (the 10-term series of the row pass)
+    double k_first = 0., k_last = 0., k_light = 0.;  // range of the row pass's K arguments (YieldArgs)
     bool light_beyond = false;  // a species below 0.7 GeV after the first nlight ones
     DBuf<char> d_rows;
     DBuf<float4> d_ecell;      // [2 Nc]: per cell flow and 3+1D position (k_emit_cells)
     DBuf<RowSp> d_rowsp;       // [2][row_stride(Ns, 4)]: all species, then negative charges suppressed
     bool charges_outside = false;  // a species charge beyond the row pass's fugacity rows
-    DBuf<double> d_cdf, d_ctot, d_partial, d_stot;
+    DBuf<RowSpD> d_rowspd;     // the same in FP64, [2][row_stride(Ns, 8)]
+    DBuf<double> d_cdf, d_ctot, d_ctot_part, d_partial, d_stot;
     DBuf<int> d_oob;
     DBuf<char> d_raw;
     // sampling
@@ -635,37 +637,66 @@ int launch_yield(iss_ctx* ctx, const YieldArgs& a, bool raw, bool exact) {
     }
 }
 
+// The row pass's items and shares.  Costs from the instruction counts, a
+// 64-byte segment of one-term species being 100; the general series takes
+// species one at a time.  Every share holds the start of at least one item
+// (the largest item costs less), so that the pieces of a tile belong to
+// consecutive waves.
+template <typename R>
+RowWork row_work(const YieldArgs& a, bool fast, int64_t waves) {
+    const int SC = row_chunk(sizeof(R)), stride = row_stride(a.Ns, sizeof(R));
+    RowWork w{};
+    w.nslow = fast ? std::min(stride, std::max(SC, (a.nlight + SC - 1) / SC * SC)) : stride;
+    w.nlight = fast ? a.nlight : 0;
+    w.nitems = w.nslow + (stride - w.nslow) / SC;
+    w.clight = sizeof(R) == 8 ? 90 : 32;
+    w.cone = fast ? (sizeof(R) == 8 ? 19 : 9) : 100;
+    w.cseg = 100;
+    w.total = (a.Nc + kWave - 1) / kWave * w.tile_cost();
+    w.waves = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(waves, w.total / 101)));
+    return w;
+}
+
 template <typename R, int MODE, bool EXACT>
-int launch_rows_t(iss_ctx* ctx, const YieldArgs& a, int max_blocks, int force_blocks) {
+int launch_rows_t(iss_ctx* ctx, YieldArgs& a, int max_blocks, int force_blocks) {
+    constexpr int kT = kRowThreads;
     const size_t lds = yield_rows_lds_bytes<R>(ktables_for(MODE), ctx->Ns);
     auto kern = k_yield_rows<R, MODE, EXACT>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             static_cast<int>(lds)) != hipSuccess)
         return ISS_ERR_HIP;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kRowThreads, lds) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    per_cu = std::min(per_cu, kPartialBlocksPerCU);  // the species partials hold num_cu * 8 blocks
-    const int64_t ntiles = (a.Nc + kRowThreads - 1) / kRowThreads;
-    // (a forced count: the same grid as an earlier pass, whose partials a
-    // skipped pass leaves in place)
-    const int nblk = force_blocks > 0 ? force_blocks
-                                      : static_cast<int>(std::max<int64_t>(
-                                            1, std::min<int64_t>({ntiles, int64_t(ctx->num_cu) * per_cu,
-                                                                  int64_t(max_blocks)})));
-    ctx->yield_grid = nblk;
-    kern<<<nblk, kRowThreads, lds, ctx->stream>>>(a, a.spk, a.rowsp);
+    if (force_blocks <= 0) {
+        // (a forced count: the same grid and groups as an earlier pass, whose
+        // partials a skipped pass leaves in place)
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kT, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+        per_cu = std::min(per_cu, kPartialBlocksPerCU);  // the species partials hold num_cu * 8 blocks
+        const int64_t most = std::min<int64_t>(int64_t(ctx->num_cu) * per_cu, max_blocks);
+        const bool fast = !EXACT && !a.all_general && !(sizeof(R) == sizeof(float) && MODE == BULK_22MOM);
+        a.work = row_work<R>(a, fast, most * (kT / kWave));
+        force_blocks = static_cast<int>(std::min<int64_t>(a.work.waves, most));
+    }
+    if (a.ctot) {
+        // a tile's pieces at most: its cost over the smallest share, one cut more
+        const int64_t pieces = a.work.tile_cost() / std::max<int64_t>(1, a.work.total / a.work.waves) + 2;
+        if (ctx->d_ctot_part.ensure(static_cast<size_t>(pieces) * a.Nc) != hipSuccess) return ISS_ERR_NOMEM;
+        a.ctot_part = ctx->d_ctot_part.p;
+    }
+    ctx->yield_grid = force_blocks;
+    const typename RowK<R>::Sp* sp;
+    if constexpr (sizeof(R) == 8) sp = a.rowspd; else sp = a.rowsp;
+    kern<<<force_blocks, kT, lds, ctx->stream>>>(a, a.spk, sp);
     return hipGetLastError() == hipSuccess ? ISS_OK : ISS_ERR_HIP;
 }
 
 template <typename R, int MODE>
-int launch_rows_m(iss_ctx* ctx, const YieldArgs& a, bool exact, int max_blocks, int force_blocks) {
+int launch_rows_m(iss_ctx* ctx, YieldArgs& a, bool exact, int max_blocks, int force_blocks) {
     return exact ? launch_rows_t<R, MODE, true>(ctx, a, max_blocks, force_blocks)
                  : launch_rows_t<R, MODE, false>(ctx, a, max_blocks, force_blocks);
 }
 
 template <typename R>
-int launch_rows(iss_ctx* ctx, const YieldArgs& a, bool exact, int max_blocks = 1 << 30, int force_blocks = 0) {
+int launch_rows(iss_ctx* ctx, YieldArgs& a, bool exact, int max_blocks = 1 << 30, int force_blocks = 0) {
     switch (a.bulk) {
         case BULK_RTA: return launch_rows_m<R, BULK_RTA>(ctx, a, exact, max_blocks, force_blocks);
         case BULK_CE: return launch_rows_m<R, BULK_CE>(ctx, a, exact, max_blocks, force_blocks);
@@ -691,7 +722,11 @@ YieldArgs base_yield_args(iss_ctx* ctx, int lcc) {
     a.spk = ctx->d_spk.p;
     a.lcc = lcc;
     a.nlight = ctx->nlight;
+    a.k_first = ctx->k_first;
+    a.k_last = ctx->k_last;
+    a.k_light = ctx->k_light;
     a.rowsp = ctx->d_rowsp.p ? ctx->d_rowsp.p + (lcc ? row_stride(Ns, 4) : 0) : nullptr;
+    a.rowspd = ctx->d_rowspd.p ? ctx->d_rowspd.p + (lcc ? row_stride(Ns, 8) : 0) : nullptr;
     a.all_general = (ctx->light_beyond || ctx->charges_outside) ? 1 : 0;
     return a;
 }
@@ -765,7 +800,9 @@ int run_yields(iss_ctx* ctx, int precision, void* per_cell_host, double* totals_
             HIPCHK(hipMemsetAsync(ctx->d_partial.p, 0, sizeof(double) * Ns, ctx->stream));
         }
         HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-        k_species_reduce<<<Ns, 256, 0, ctx->stream>>>(ctx->d_partial.p, nblk, Ns, ctx->d_stot.p);
+        const int cblk = a.ctot_part ? static_cast<int>((Nc + 255) / 256) : 0;
+        k_species_reduce<<<Ns + cblk, 256, 0, ctx->stream>>>(ctx->d_partial.p, nblk, Ns, ctx->d_stot.p, a.ctot_part,
+                                                             a.work, Nc, ctx->d_ctot.p);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
         const bool check = Nc > 0 && !exact;
@@ -1078,7 +1115,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_ktab.release(); ctx->d_ktabf.release(); ctx->d_ptab.release();
     ctx->d_cells.release(); ctx->d_tmp.release(); ctx->d_lab.release(); ctx->d_coef.release(); ctx->d_u32.release();
     ctx->d_i64.release(); ctx->d_mu_used.release(); ctx->d_scan.release(); ctx->d_eos.release(); ctx->d_cdf.release();
-    ctx->d_ctot.release(); ctx->d_partial.release(); ctx->d_oob.release(); ctx->d_stot.release(); ctx->d_raw.release();
+    ctx->d_ctot.release(); ctx->d_ctot_part.release(); ctx->d_rowspd.release(); ctx->d_partial.release(); ctx->d_oob.release(); ctx->d_stot.release(); ctx->d_raw.release();
     ctx->d_counts.release(); ctx->d_evcount.release(); ctx->d_off.release(); ctx->d_evoff.release();
     ctx->d_tree0.release(); ctx->d_tree1.release(); ctx->d_out.release(); ctx->d_setup.release(); ctx->d_stats.release();
     ctx->d_cellidx.release(); ctx->d_ecell.release();
@@ -1195,6 +1232,31 @@ int iss_set_species(iss_ctx* ctx, const iss_species_desc* sp) {
             }
         HIPCHK(ctx->d_rowsp.ensure(rs.size()));
         HIPCHK(hipMemcpy(ctx->d_rowsp.p, rs.data(), sizeof(RowSp) * rs.size(), hipMemcpyHostToDevice));
+        const int std_ = row_stride(Ns, 8);
+        std::vector<RowSpD> rd(2 * static_cast<size_t>(std_));
+        for (int v = 0; v < 2; v++)
+            for (int i = 0; i < std_; i++) {
+                const RowSp& f = rs[static_cast<size_t>(v) * st + i];
+                const double m = i < Ns ? sp->mass[i] : 1.0, m2 = m * m;
+                // (a charge outside the rows: the pass takes the general series)
+                const int B = i < Ns ? sp->baryon[i] : 0, S = i < Ns ? sp->strange[i] : 0, Q = i < Ns ? sp->charge[i] : 0;
+                auto off = [&](int kind, int q) {
+                    return ctx->charges_outside ? 0 : fug_row_d(kind, q) * kRowThreads * static_cast<int>(sizeof(double));
+                };
+                rd[static_cast<size_t>(v) * std_ + i] =
+                    RowSpD{20. * m, m2, 3. * m2 * B, m2 * m * B, m2 * m, m2 * m2, f.g, off(0, B), off(1, S), off(2, Q),
+                           f.sgn, static_cast<double>(B), static_cast<double>(S), static_cast<double>(Q)};
+            }
+        // the K arguments' range (n m / T) over all items, the padding's included
+        ctx->k_first = ctx->k_last = 20.;
+        ctx->k_light = 0.;
+        for (int i = 0; i < Ns; i++) {
+            ctx->k_first = std::min(ctx->k_first, 20. * sp->mass[i]);
+            ctx->k_last = std::max(ctx->k_last, 20. * sp->mass[i]);
+            if (i < ctx->nlight) ctx->k_light = std::max(ctx->k_light, 200. * sp->mass[i]);
+        }
+        HIPCHK(ctx->d_rowspd.ensure(rd.size()));
+        HIPCHK(hipMemcpy(ctx->d_rowspd.p, rd.data(), sizeof(RowSpD) * rd.size(), hipMemcpyHostToDevice));
     }
     ctx->h_pid.assign(sp->pid, sp->pid + Ns);
     ctx->h_sp.resize(Ns);
@@ -1411,7 +1473,7 @@ int iss_compute_yields_noalloc(iss_ctx* ctx, const iss_yield_opts* opts, double*
             nblk = ctx->yield_grid;
         }
     }
-    k_species_reduce<<<Ns, 256, 0, ctx->stream>>>(partial, nblk, Ns, species_totals);
+    k_species_reduce<<<Ns, 256, 0, ctx->stream>>>(partial, nblk, Ns, species_totals, nullptr, RowWork{}, 0, nullptr);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return ISS_OK;

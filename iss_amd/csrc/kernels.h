@@ -80,6 +80,36 @@ struct RowSp {
 };
 static_assert(sizeof(RowSp) == 40 && alignof(RowSp) == 8, "RowSp is copied to LDS as 10 words");
 
+// the same for the FP64 row pass: the products of powers of m and B that its
+// K coefficients are linear in, byte offsets of the fugacity rows, and the
+// charges (22-moment bulk)
+struct RowSpD {
+    double md20, m2, m2B3, m3B, m3, m4, g;   // m2B3 = 3 m^2 B
+    int fB, fS, fQ;
+    float sgn;
+    double B, S, Q;
+};
+
+// The row pass's work: every 64-cell tile is a row of items (single species
+// of the leading segments, then whole segments) with integer costs, and wave
+// w of `waves` takes the items that start in its share [w total / waves,
+// (w + 1) total / waves) of all tiles' costs, tile after tile.
+struct RowWork {
+    int64_t total;           // tiles x cost of a tile
+    int waves;
+    int nitems, nslow, nlight;   // items: nslow single species (nlight of them light), then segments
+    int clight, cone, cseg;      // their costs
+    __host__ __device__ int start(int i) const {   // cost before item i
+        if (i <= nlight) return i * clight;
+        if (i <= nslow) return nlight * clight + (i - nlight) * cone;
+        return nlight * clight + (nslow - nlight) * cone + (i - nslow) * cseg;
+    }
+    __host__ __device__ int tile_cost() const { return start(nitems); }
+    __host__ __device__ int64_t share(int64_t w) const { return w * total / waves; }
+    // the wave whose share holds cost x
+    __host__ __device__ int64_t owner(int64_t x) const { return ((x + 1) * waves - 1) / total; }
+};
+
 struct PTabDev {
     // per table: first E~, step, length, m0, truncation, fermion flag
     double Et0[6], dEt[6], m0[6];
@@ -108,7 +138,12 @@ struct YieldArgs {
     int lcc;              // local charge conservation: negative species get no yield
     double* ycol;         // optional [Ns][Nc] FP64 yields, species-major (multiplicity models)
     void* rows;           // k_yield_rows: [Nc][row stride] yields in working precision, cell-major
-    const struct RowSp* rowsp;  // k_yield_rows: species constants, padded (zero weight beyond Ns)
+    const struct RowSp* rowsp;   // k_yield_rows: species constants, padded (zero weight beyond Ns)
+    const struct RowSpD* rowspd;  // the same in FP64
+    double k_first, k_last, k_light;  // k_yield_rows: 20 x (smallest, largest n m) of the one-term items, and
+                                      // 200 x the heaviest light species' mass (0: none)
+    RowWork work;                // k_yield_rows: how the waves share the items
+    double* ctot_part;           // [pieces][Nc] cell totals of a tile's pieces, in wave order
     int nlight;           // k_yield_rows: leading species below 0.7 GeV (the 10-term series)
     int all_general;      // k_yield_rows: a species below 0.7 GeV after the leading ones (at most 16),
                           // or a charge outside the fugacity rows: every species takes the general series

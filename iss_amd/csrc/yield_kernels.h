@@ -428,10 +428,23 @@ __global__ void k_clear_flag(int* flag) {
     if (threadIdx.x == 0) *flag = 0;
 }
 
+// (workgroups past the species add the cell totals of each tile's pieces, in
+// wave order)
 __global__ void k_species_reduce(const double* __restrict__ partial, int nblk, int Ns,
-                                 double* __restrict__ out) {
+                                 double* __restrict__ out, const double* __restrict__ ctot_part, RowWork work,
+                                 int64_t Nc, double* __restrict__ ctot) {
     __shared__ double red[256];
     const int s = blockIdx.x;
+    if (s >= Ns) {
+        const int64_t c = static_cast<int64_t>(s - Ns) * blockDim.x + threadIdx.x;
+        if (c >= Nc) return;
+        const int64_t x = c / kWave * work.tile_cost();
+        const int64_t pieces = work.owner(x + work.start(work.nitems - 1)) - work.owner(x) + 1;
+        double t = ctot_part[c];
+        for (int64_t g = 1; g < pieces; g++) t += ctot_part[g * Nc + c];
+        ctot[c] = t;
+        return;
+    }
     double v = 0.;
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) v += partial[static_cast<int64_t>(b) * Ns + s];
     red[threadIdx.x] = v;
@@ -504,30 +517,37 @@ __global__ void k_diffusion_dn(YieldArgs a, const double* __restrict__ etab, dou
 // FP64 species partials.  The sampling pass builds each cell's FP64 species
 // CDF from its row when it picks species (k_pick), so no CDF is stored.
 //
-// One cell per thread, tiles of 256 cells (persistent over tiles); the
-// species loop is uniform across the workgroup, a 64-byte segment of species
-// at a time:
-//   * the species constants come from a padded table staged in LDS
-//     (broadcast reads that wait in order with the K reads);
-//   * FP32, one-term species (above 0.7 GeV): the fugacity is a product of
-//     per-cell powers e^{beta mu q} picked by the species' charges, the K
-//     table position t = 20 m / T - 10 is one FP64 fma, and the 14-moment
-//     (or RTA / Chapman-Enskog / 22-moment) bulk terms are formed from
+// One cell per thread, 64 cells per wave.  A wave takes an equal share of the
+// pass's cost, tile after tile (RowWork): with fixed tiles per wave the last
+// round of tiles left up to half of the chip idle, and a surface of few tiles
+// all but those tiles' CUs.  A tile may be split between waves; its cell
+// totals are then added in wave order by k_species_reduce.  The species loop
+// is uniform across the wave, a 64-byte segment of species at a time:
+//   * the species constants come from a padded table: FP32 from LDS (broadcast
+//     reads that wait in order with the K reads), FP64 by scalar loads (80 bytes
+//     a species: as LDS broadcasts they were half of the pass's LDS time);
+//   * one-term species (above 0.7 GeV): the fugacity is a product of per-cell
+//     powers e^{beta mu q} picked by the species' charges, the K table
+//     position t = 20 m / T - 10 is one FP64 fma, and the 14-moment (or RTA /
+//     Chapman-Enskog, in FP64 also 22-moment) bulk terms are formed from
 //     per-cell products, all with lambda factored out (the same sums as the
 //     general series with n = 1);
-//   * FP32, light species (the leading ones below 0.7 GeV): the same ten
-//     terms as the general series, unrolled;
+//   * light species (the leading ones below 0.7 GeV): the same ten terms as
+//     the general series, unrolled;
 //   * diffusion: the per-item correction is added to either;
-//   * FP64 mode, the exact-K rerun, 22-moment bulk delta f and
-//     species lists outside these assumptions take the general series
-//     (yield_one);
-//   * items whose terms cancel beyond kIllCond are recomputed in FP64, 64
+//   * the exact-K rerun, FP32 22-moment bulk delta f and species lists outside
+//     these assumptions take the general series (yield_one);
+//   * FP32 items whose terms cancel beyond kIllCond are recomputed in FP64, 64
 //     at a time from a per-wave queue (one item per lane);
 //   * each thread stores its segment with 16-byte stores (whole 64-byte
 //     sectors), adds the yields to its FP64 cell total in species order, and
 //     the species' FP64 sums over the wave's 64 cells come from DPP
 //     reductions, accumulated per wave in LDS (a fixed order).
-constexpr int kRowThreads = 256;
+// LDS holds one workgroup per CU: the K rows (and species table) once for its
+// 12 waves.  Measured: FP64, 200,000 cells 974 -> 269 us (LDS busy 62 %, of that
+// half conflicts of the K rows; VALU 45 %), 2000 cells 237 -> 20 us; FP32, 1e6
+// cells 1263 -> 1065 us (VALU 80 %), 200,000 323 -> 260 us.
+constexpr int kRowThreads = 768;
 constexpr int kKRows = 1024;     // K rows staged in LDS (arguments below 51.7)
 constexpr int kLightMax = 16;
 
@@ -541,10 +561,12 @@ __host__ __device__ constexpr int row_stride(int ns, int esz) {
 template <typename R>
 struct RowK {
     using T = double;
+    using Sp = RowSpD;
 };
 template <>
 struct RowK<float> {
     using T = float2;
+    using Sp = RowSp;
 };
 
 template <bool EXACT>
@@ -560,6 +582,20 @@ struct KLookupRows32 {
         } else {
             at<NK>((arg - kKx0) * 20.0, K2, K1, K3);
         }
+    }
+    // at table position t = (x - 0.5) / 0.05 known to lie in the staged rows
+    // (rows_inside); any t stays inside them
+    template <int NK>
+    __device__ __forceinline__ void inside(double t, float& K2, float& K1, float& K3) const {
+        const uint32_t idx = min(static_cast<uint32_t>(static_cast<int>(t)), static_cast<uint32_t>(kKRows - 2));
+        const float fr = static_cast<float>(t - static_cast<double>(static_cast<int>(idx)));
+        const float2 v2 = lds[idx];
+        float2 v1 = make_float2(0.f, 0.f), v3 = make_float2(0.f, 0.f);
+        if (NK >= 2) v1 = lds[kKRows + idx];
+        if (NK >= 3) v3 = lds[2 * kKRows + idx];
+        K2 = fmaf(fr, v2.y, v2.x);
+        if (NK >= 2) K1 = fmaf(fr, v1.y, v1.x);
+        if (NK >= 3) K3 = fmaf(fr, v3.y, v3.x);
     }
     // the same at table position t = (x - 0.5) / 0.05
     template <int NK>
@@ -655,20 +691,29 @@ __device__ __forceinline__ void row_cell_f(const YieldArgs& a, int64_t c, bool v
     }
 }
 
+// Whether every K argument of a cell lies in the staged rows: the table
+// position grows with the argument, so its smallest and largest items decide
+// (NaN and negative temperatures fail).  One test per cell instead of one per
+// item.
+__device__ __forceinline__ bool rows_inside(const YieldArgs& a, double T, double beta) {
+    const double t0 = fma(a.k_first, beta, -10.0), t1 = fma(a.k_last, beta, -10.0);
+    const double t2 = (a.k_light > 0. && T > 0.05) ? fma(a.k_light, beta, -10.0) : t1;
+    return t0 >= 0. && t1 < kKRows - 1 && t2 < kKRows - 1;
+}
+
 // FP32 yield of a one-term species (n = 1) from the padded species table:
 // the general series' sums with lambda factored out, branch-free: the
 // fugacity is the product of three per-cell factors read from the thread's
 // LDS column (rows picked by the species' charges), K from the staged rows.
-// Returns the unclamped yield; ill: the terms cancel beyond kIllCond; ok: the
-// K argument lies in the staged rows.
+// Returns the unclamped yield; ill: the terms cancel beyond kIllCond.
 template <int MODE>
 __device__ __forceinline__ float row_yield_sp(const RowSp& q, const RowCellF& p, const float* fug,
-                                              const KLookupRows32<false>& kl, bool& ill, bool& ok) {
+                                              const KLookupRows32<false>& kl, bool& ill) {
     float K2 = 0.f, K1 = 0.f, K3 = 0.f;
     constexpr int NK = (MODE == BULK_NONE) ? 1 : ((MODE == BULK_RTA || MODE == BULK_CE) ? 2 : 3);
-    ok = kl.template at_ok<NK>(fma(q.md20, p.betad, -10.0), K2, K1, K3);
-    const float lam = fug[(q.frow & 0xFF) * kRowThreads] * fug[((q.frow >> 8) & 0xFF) * kRowThreads] *
-                      fug[(q.frow >> 16) * kRowThreads];
+    kl.template inside<NK>(fma(q.md20, p.betad, -10.0), K2, K1, K3);
+    constexpr int kT = kRowThreads;
+    const float lam = fug[(q.frow & 0xFF) * kT] * fug[((q.frow >> 8) & 0xFF) * kT] * fug[(q.frow >> 16) * kT];
     const float a0 = (q.m2 * p.T) * K2;
     float br = a0;
     ill = false;
@@ -692,25 +737,23 @@ __device__ __forceinline__ float row_yield_sp(const RowSp& q, const RowCellF& p,
 // terms (one where T <= 0.05 GeV), unrolled so that their K reads are in
 // flight together; lambda from the fugacity column, the constants from the
 // padded table (sgn: +1 fermions, -1 bosons).  Returns the unclamped yield;
-// ill and ok as row_yield_sp.
+// ill as row_yield_sp.
 constexpr int kLightTerms = 10;
 template <int MODE>
 __device__ __forceinline__ float row_yield_light(const RowSp& q, const RowCellF& p, const float* fug,
-                                                 const KLookupRows32<false>& kl, bool& ill, bool& ok) {
+                                                 const KLookupRows32<false>& kl, bool& ill) {
     constexpr int NK = (MODE == BULK_NONE) ? 1 : ((MODE == BULK_RTA || MODE == BULK_CE) ? 2 : 3);
-    const float lam = fug[(q.frow & 0xFF) * kRowThreads] * fug[((q.frow >> 8) & 0xFF) * kRowThreads] *
-                      fug[(q.frow >> 16) * kRowThreads];
+    constexpr int kT = kRowThreads;
+    const float lam = fug[(q.frow & 0xFF) * kT] * fug[((q.frow >> 8) & 0xFF) * kT] * fug[(q.frow >> 16) * kT];
     const float more = p.T > 0.05f ? 1.f : 0.f;  // weight of the terms beyond the first
     const float mb = q.m * p.beta;
     float r0 = 0.f, r1 = 0.f, r2 = 0.f, r3 = 0.f;
     float th = 1.f, fl = lam;
-    ok = true;
 #pragma unroll
     for (int n = 1; n <= kLightTerms; n++) {
         float K2 = 0.f, K1 = 0.f, K3 = 0.f;
-        const bool okn = kl.template at_ok<NK>(fma(static_cast<double>(n) * q.md20, p.betad, -10.0), K2, K1, K3);
+        kl.template inside<NK>(fma(static_cast<double>(n) * q.md20, p.betad, -10.0), K2, K1, K3);
         const float w = n == 1 ? 1.f : more;
-        ok = ok && (okn || w == 0.f);
         const float inv = 1.f / static_cast<float>(n);
         const float thn = th * inv, k2n = 3.f * K2 * inv, tf = w * (th * fl);
         r0 += w * (thn * fl * K2);
@@ -742,23 +785,136 @@ __device__ __forceinline__ float row_yield_light(const RowSp& q, const RowCellF&
     return Neq;
 }
 
+// ---- FP64: the same sums with each cell's products folded into the factors
+// of m^a B^b that multiply K_1, K_2 and K_3, so that an item is one table
+// position, three interpolations and 15 products (the general series: 120
+// FP64 instructions, a fifth of them in divisions).
+// per-cell quantities: 1 / T, T, the prefactor dsigma_0 / (2 pi^2 (hbar c)^3) and
+// the factors k* (MODE-dependent)
+struct RowCellD {
+    double beta, T, pdc, k4, kB, k3B, k3, kS, kQ;
+};
+
+template <int MODE>
+__device__ __forceinline__ void row_cell_d(const YieldArgs& a, int64_t c, bool valid, RowCellD& p, double mu[3]) {
+    const int64_t Nc = a.Nc;
+    p.T = 0.15;
+    double dsu = 0., Pi = 0.;
+    double cf[6] = {0., 0., 0., 0., 0., 0.};
+    mu[0] = mu[1] = mu[2] = 0.;
+    if (valid) {
+        p.T = a.cells[F_T * Nc + c];
+        mu[0] = a.cells[F_MUB * Nc + c];
+        mu[1] = a.cells[F_MUS * Nc + c];
+        mu[2] = a.cells[F_MUQ * Nc + c];
+        dsu = a.cells[F_DA0 * Nc + c];
+        if (MODE != BULK_NONE) {
+            Pi = a.cells[F_PI * Nc + c];
+            if (MODE == BULK_RTA) Pi = Pi / kHbarC;
+#pragma unroll
+            for (int k = 0; k < 6; k++) cf[k] = a.coef[k * Nc + c];
+        }
+    }
+    p.beta = 1. / p.T;
+    p.pdc = dsu * (1.0 / (kHbarC * kHbarC * kHbarC) / (2. * kPi * kPi));
+    const double T2 = p.T * p.T;
+    p.k4 = p.kB = p.k3B = p.k3 = p.kS = p.kQ = 0.;
+    // the series' terms: m^2 T K2 / n + Pi times, with x = m / T,
+    //   RTA, CE:    c0 c1 T m^2 (x K1 + 3 K2 / n) - c0 m^3 / 3 K1
+    //   14-moment:  c0 T m^4 K2 + c1 T^2 m^2 B (x K1 + 3 K2 / n) + c2 T^2 m^3 (x K2 + 3 K3 / n)
+    //   22-moment:  c2 for c0, B c3 + S c4 + Q c5 for B c1, c1 - c2 for c2
+    if (MODE == BULK_RTA || MODE == BULK_CE) {
+        const double k = Pi * cf[0] * cf[1] * p.T;
+        p.kB = 3. * k;
+        p.k3 = k * p.beta - Pi * cf[0] / 3.;
+    } else if (MODE == BULK_14MOM || MODE == BULK_22MOM) {
+        const bool m22 = MODE == BULK_22MOM;
+        const double q = Pi * T2 * (m22 ? cf[1] - cf[2] : cf[2]);
+        p.k4 = Pi * p.T * (m22 ? cf[2] : cf[0]) + q * p.beta;
+        p.k3 = 3. * q;
+        p.kB = Pi * T2 * (m22 ? cf[3] : cf[1]);
+        p.k3B = p.kB * p.beta;
+        if (m22) {
+            p.kS = Pi * T2 * cf[4];
+            p.kQ = Pi * T2 * cf[5];
+        }
+    }
+}
+
+// The series of one species in FP64, TERMS terms (1, or 10 for the light
+// species, of which those beyond the first count where T > 0.05 GeV); q: its
+// constants (scalar loads), fug: the thread's column of fugacity factors.
+// Returns the unclamped yield.
+template <int MODE, int TERMS>
+__device__ __forceinline__ double row_yield_d(const RowSpD& q, const RowCellD& p, const char* fug,
+                                              const double* s_k) {
+    constexpr int NK = ktables_for(MODE);
+    const double lam = *reinterpret_cast<const double*>(fug + q.fB) * *reinterpret_cast<const double*>(fug + q.fS) *
+                       *reinterpret_cast<const double*>(fug + q.fQ);
+    // K2 takes c2 / n + c2n, K1 c1, K3 c3 / n
+    double c2 = q.m2 * p.T, c2n = 0., c1 = 0., c3 = 0.;
+    if (MODE == BULK_RTA || MODE == BULK_CE) {
+        c2 = fma(q.m2, p.kB, c2);
+        c1 = q.m3 * p.k3;
+    } else if (MODE == BULK_14MOM) {
+        c2 = fma(q.m2B3, p.kB, c2);
+        c1 = q.m3B * p.k3B;
+    } else if (MODE == BULK_22MOM) {
+        const double u = q.B * p.kB + q.S * p.kS + q.Q * p.kQ;
+        c2 = fma(3. * q.m2, u, c2);
+        c1 = q.m3 * (u * p.beta);
+    }
+    if (MODE == BULK_14MOM || MODE == BULK_22MOM) {
+        c2n = q.m4 * p.k4;
+        c3 = q.m3 * p.k3;
+    }
+    double sum = 0., w = 1.;
+#pragma unroll
+    for (int n = 1; n <= TERMS; n++) {
+        const double t = fma(n == 1 ? q.md20 : n * q.md20, p.beta, -10.0);
+        const uint32_t idx = min(static_cast<uint32_t>(static_cast<int>(t)), static_cast<uint32_t>(kKRows - 2));
+        const double fr = t - static_cast<double>(static_cast<int>(idx));
+        const double* k = s_k + NK * idx;   // (rows of K_2, K_1, K_3)
+        const double inv = 1. / n;
+        double v = (n == 1 ? c2 + c2n : fma(c2, inv, c2n)) * fma(fr, k[NK] - k[0], k[0]);
+        if (NK >= 2) v = fma(c1, fma(fr, k[NK + 1] - k[1], k[1]), v);
+        if (NK >= 3) v = fma(n == 1 ? c3 : c3 * inv, fma(fr, k[NK + 2] - k[2], k[2]), v);
+        if (n == 1) {
+            sum = v;
+            w = p.T > 0.05 ? -static_cast<double>(q.sgn) * lam : 0.;
+        } else {
+            sum = fma(w, v, sum);
+            w *= -static_cast<double>(q.sgn) * lam;
+        }
+    }
+    return (q.g * p.pdc) * lam * sum;
+}
+
 // fugacity rows of the LDS column: e^{beta mu_B q}, q = -1..1; e^{beta mu_S q},
 // q = -3..3; e^{beta mu_Q q}, q = -2..2
-constexpr int kFugRows = 15;
+// (FP32); the FP64 column holds 1 once, for every charge 0, and the other
+// charges' factors (fug_row_d)
+constexpr int kFugRows = 15, kFugRowsD = 13;
+__host__ __device__ constexpr int fug_row_d(int kind, int q) {
+    return q == 0 ? 0 : kind == 0 ? (q < 0 ? 1 : 2) : kind == 1 ? (q < 0 ? q + 6 : q + 5) : (q < 0 ? q + 11 : q + 10);
+}
 
 template <typename R>
 __host__ __device__ constexpr size_t yield_rows_lds_bytes(int ntab, int ns) {
+    constexpr int kT = kRowThreads;
     return static_cast<size_t>(ntab) * kKRows * sizeof(typename RowK<R>::T)               // K rows
-           + static_cast<size_t>(kRowThreads / kWave) * row_stride(ns, sizeof(R)) * sizeof(double)   // wave sums
-           + (sizeof(R) == sizeof(float)  // fugacities, the padded species table, the FP64 queues
-                  ? static_cast<size_t>(kFugRows) * kRowThreads * sizeof(float) + row_stride(ns, 4) * sizeof(RowSp) +
-                        static_cast<size_t>(kRowThreads) * (sizeof(double) + sizeof(int) + sizeof(float))
+           + static_cast<size_t>(kT / kWave) * row_stride(ns, sizeof(R)) * sizeof(double)   // wave sums
+           + static_cast<size_t>(sizeof(R) == 8 ? kFugRowsD : kFugRows) * kT * sizeof(R)  // fugacities
+           + (sizeof(R) == sizeof(float)  // FP32: the padded species table, the FP64 queues
+                  ? row_stride(ns, 4) * sizeof(RowSp) + kT * (sizeof(double) + sizeof(int) + sizeof(float))
                   : 0);
 }
+static_assert(yield_rows_lds_bytes<float>(3, kMaxSpecies) <= 160 * 1024, "FP32 rows: one workgroup per CU");
+static_assert(yield_rows_lds_bytes<double>(3, kMaxSpecies) <= 160 * 1024, "FP64 rows: one workgroup per CU");
 
 template <typename R, int MODE, bool EXACT>
-__global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const SpeciesK* __restrict__ spk,
-                                                            const RowSp* __restrict__ rowsp) {
+__global__ __launch_bounds__(kRowThreads) void k_yield_rows(
+    YieldArgs a, const SpeciesK* __restrict__ spk, const typename RowK<R>::Sp* __restrict__ rowsp) {
     // the exact-K pass after a first pass that stayed inside the staged rows:
     // nothing to redo (uniform over the grid; the flag only ever turns on)
     if (EXACT && a.gate && *a.gate == 0) return;
@@ -767,22 +923,27 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
     constexpr int NT = ktables_for(MODE);
     constexpr int SC = row_chunk(sizeof(R));
     constexpr bool F32 = sizeof(R) == sizeof(float);
+    constexpr int kT = kRowThreads;
+    using Sp = typename RowK<R>::Sp;
     const int Ns = a.Ns, L = a.nlight, stride = row_stride(Ns, sizeof(R));
-    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    // (FP64: the wave index as a scalar, for scalar loads of the species'
+    // constants; FP32 has them in LDS and is faster without the scalars)
+    const int w = F32 ? threadIdx.x / kWave : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int lane = threadIdx.x % kWave;
     KT* s_k = reinterpret_cast<KT*>(smem);
     double* s_acc = reinterpret_cast<double*>(s_k + NT * kKRows);  // [waves][stride]
-    float* s_fug = reinterpret_cast<float*>(s_acc + (kRowThreads / kWave) * stride);  // [kFugRows][threads]
-    float* fug = s_fug + threadIdx.x;
+    R* s_fug = reinterpret_cast<R*>(s_acc + (kT / kWave) * stride);  // [kFugRows][threads]
+    R* fug = s_fug + threadIdx.x;
     // the padded species table: broadcast LDS reads, in order with the K and
     // fugacity reads (scalar loads would share their wait counter out of order)
-    RowSp* s_sp = reinterpret_cast<RowSp*>(s_fug + kFugRows * kRowThreads);
+    Sp* s_sp = reinterpret_cast<Sp*>(s_fug + kFugRows * kT);
     // the wave's queue of items to recompute in FP64
-    double* q_d = reinterpret_cast<double*>(s_sp + (F32 ? row_stride(Ns, 4) : 0)) + w * kWave;
-    int* q_key = reinterpret_cast<int*>(q_d - w * kWave + kRowThreads) + w * kWave;
-    float* q_old = reinterpret_cast<float*>(q_key - w * kWave + kRowThreads) + w * kWave;
+    double* q_d = reinterpret_cast<double*>(s_sp + stride) + w * kWave;
+    int* q_key = reinterpret_cast<int*>(q_d - w * kWave + kT) + w * kWave;
+    float* q_old = reinterpret_cast<float*>(q_key - w * kWave + kT) + w * kWave;
     R* rows = static_cast<R*>(a.rows);
     if (F32 && rowsp) {
-        const int n = row_stride(Ns, 4) * static_cast<int>(sizeof(RowSp) / sizeof(int));
+        const int n = stride * static_cast<int>(sizeof(Sp) / sizeof(int));
         const int* src = reinterpret_cast<const int*>(rowsp);
         int* dstp = reinterpret_cast<int*>(s_sp);
         for (int i = threadIdx.x; i < n; i += blockDim.x) dstp[i] = src[i];
@@ -793,17 +954,32 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
             const int t = i / kKRows, r = i % kKRows;
             const int o = (t == 0) ? 2 : (t == 1 ? 1 : 3);
             if constexpr (F32) s_k[i] = a.ktabf[(o - 1) * kKLen + r];
-            else s_k[i] = a.ktab[(o - 1) * kKLen + r];
+            // (FP64 fast path: one row of all orders; the general series: one table per order)
+            else s_k[a.all_general ? i : NT * r + t] = a.ktab[(o - 1) * kKLen + r];
         }
     }
-    for (int i = threadIdx.x; i < (kRowThreads / kWave) * stride; i += blockDim.x) s_acc[i] = 0.;
+    for (int i = threadIdx.x; i < (kT / kWave) * stride; i += blockDim.x) s_acc[i] = 0.;
     __syncthreads();
     double* wacc = s_acc + w * stride;
 
     const int64_t Nc = a.Nc;
-    const int64_t ntiles = (Nc + kRowThreads - 1) / kRowThreads;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t c = tile * kRowThreads + threadIdx.x;
+    // consecutive shares go to different workgroups, so that few waves spread
+    // over the CUs
+    const RowWork& wk = a.work;
+    const int64_t wid = static_cast<int64_t>(w) * gridDim.x + blockIdx.x;
+    const int64_t lo = wid < wk.waves ? wk.share(wid) : wk.total, hi = wid < wk.waves ? wk.share(wid + 1) : wk.total;
+    const int tcost = wk.tile_cost();
+    for (int64_t tile = lo / tcost; tile * tcost < hi; tile++) {
+        // the tile's items that start inside [lo, hi)
+        int ibeg = 0, iend = wk.nitems;
+        while (ibeg < wk.nitems && tile * tcost + wk.start(ibeg) < lo) ibeg++;
+        while (iend > ibeg && tile * tcost + wk.start(iend - 1) >= hi) iend--;
+        if (ibeg == iend) continue;
+        // items as species: single ones below nslow, then segments
+        const int nslow = wk.nslow;
+        const int sbeg = ibeg < nslow ? ibeg : nslow + (ibeg - nslow) * SC;
+        const int send = iend <= nslow ? iend : nslow + (iend - nslow) * SC;
+        const int64_t c = tile * kWave + lane;
         const bool valid = c < Nc;
         // the cell's parameters for the general series (working precision)
         R T = R(0.15), muB = 0, muS = 0, muQ = 0, dsu = 0, Pi = 0;
@@ -860,7 +1036,7 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
         // every species on the general path, one at a time with word stores
         auto one_by_one = [&]() {
 #pragma unroll 1
-            for (int s = 0; s < stride; s++) {
+            for (int s = sbeg; s < send; s++) {
                 const R v = s < Ns ? general(s) : R(0);
                 if (valid) row[s] = v;
                 ctot += static_cast<double>(v);
@@ -868,22 +1044,22 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
                 if (lane == 0) wacc[s] += t;
             }
         };
-        // (the 22-moment bulk terms take the general series)
+        // (the FP32 22-moment bulk terms take the general series)
         bool fast = false;
-        if constexpr (F32 && !EXACT && MODE != BULK_22MOM) fast = !a.all_general && a.rowsp;
+        if constexpr (!EXACT && (!F32 || MODE != BULK_22MOM)) fast = !a.all_general && rowsp;
         if constexpr (F32 && !EXACT && MODE != BULK_22MOM) if (fast) {
             {
                 const double xb = pf.betad * static_cast<double>(muB), xs = pf.betad * static_cast<double>(muS),
                              xq = pf.betad * static_cast<double>(muQ);
 #pragma unroll
-                for (int q = -1; q <= 1; q++) fug[(q + 1) * kRowThreads] = static_cast<float>(exp(q * xb));
+                for (int q = -1; q <= 1; q++) fug[(q + 1) * kT] = static_cast<float>(exp(q * xb));
 #pragma unroll
-                for (int q = -3; q <= 3; q++) fug[(q + 6) * kRowThreads] = static_cast<float>(exp(q * xs));
+                for (int q = -3; q <= 3; q++) fug[(q + 6) * kT] = static_cast<float>(exp(q * xs));
 #pragma unroll
-                for (int q = -2; q <= 2; q++) fug[(q + 12) * kRowThreads] = static_cast<float>(exp(q * xq));
+                for (int q = -2; q <= 2; q++) fug[(q + 12) * kT] = static_cast<float>(exp(q * xq));
             }
             const KLookupRows32<false> kl1{reinterpret_cast<const float2*>(s_k), a.ktabf, a.oob};
-            bool bad = false;  // a K argument beyond the staged rows
+            const bool bad = !rows_inside(a, T, pf.betad);  // a K argument beyond the staged rows
             // the diffusion correction of (c, s) joins the terms that may
             // cancel (zero weight: none)
             const double* dnq_row = (a.dnq && valid) ? a.dnq + c * Ns : nullptr;
@@ -903,7 +1079,7 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
                 wave_lds_sync();
                 if (lane < qn) {
                     const int key = q_key[lane];
-                    const int64_t cc = tile * kRowThreads + w * kWave + (key & (kWave - 1));
+                    const int64_t cc = tile * kWave + (key & (kWave - 1));
                     const int s = key >> 6;
                     const float v = yield_fp64_cold<MODE, EXACT>(a, cc, s);
                     // after the FP32 store of the same entry by this wave
@@ -924,10 +1100,9 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
             };
             // the first segment: the light species (ten-term series), then
             // one-term species, one at a time with word stores
-            auto first = [&](int s, float v, bool ill, bool ok, const RowSp& q) {
+            auto first = [&](int s, float v, bool ill, const RowSp& q) {
                 if (a.dnq) add_dnq(s, q, v, ill);
-                bad |= !ok;
-                v = v > 0.f ? v : 0.f;
+                v = fmaxf(v, 0.f);
                 if (valid) row[s] = v;
                 ctot += static_cast<double>(v);
                 const double t = wave_sum_dpp(static_cast<double>(v));
@@ -948,34 +1123,33 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
                 }
             };
 #pragma unroll 1
-            for (int s = 0; s < L; s++) {
+            for (int s = sbeg; s < min(min(L, nslow), send); s++) {
                 const RowSp q = s_sp[s];
-                bool ill = false, ok = true;
-                const float v = row_yield_light<MODE>(q, pf, fug, kl1, ill, ok);
-                first(s, v, ill, ok, q);
+                bool ill = false;
+                const float v = row_yield_light<MODE>(q, pf, fug, kl1, ill);
+                first(s, v, ill, q);
             }
 #pragma unroll 1
-            for (int s = L; s < SC; s++) {
+            for (int s = max(L, sbeg); s < min(nslow, send); s++) {
                 const RowSp q = s_sp[s];
-                bool ill = false, ok = true;
-                const float v = row_yield_sp<MODE>(q, pf, fug, kl1, ill, ok);
-                first(s, v, ill, ok, q);
+                bool ill = false;
+                const float v = row_yield_sp<MODE>(q, pf, fug, kl1, ill);
+                first(s, v, ill, q);
             }
             // the one-term species, a 64-byte segment at a time, from the
             // padded table (zero weight beyond Ns and for suppressed
             // species; lanes of cells beyond the surface have dsigma = 0)
-            for (int s0 = SC; s0 < stride; s0 += SC) {
+            for (int s0 = max(sbeg, nslow); s0 < send; s0 += SC) {
                 float y[SC];
                 uint32_t illm = 0u;  // items to recompute in FP64
 #pragma unroll
                 for (int j = 0; j < SC; j++) {
                     const RowSp q = s_sp[s0 + j];
-                    bool ill = false, ok = true;
-                    float v = row_yield_sp<MODE>(q, pf, fug, kl1, ill, ok);
+                    bool ill = false;
+                    float v = row_yield_sp<MODE>(q, pf, fug, kl1, ill);
                     if (a.dnq) add_dnq(s0 + j, q, v, ill);
-                    v = v > 0.f ? v : 0.f;
+                    v = fmaxf(v, 0.f);
                     illm |= (ill && q.g != 0.f) ? (1u << j) : 0u;
-                    bad |= !ok;
                     y[j] = v;
                     ctot += static_cast<double>(v);
                 }
@@ -1024,13 +1198,64 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(YieldArgs a, const S
             flush();
             if (__any(bad && valid) && lane == 0) *a.oob = 1;
         }
+        if constexpr (!F32 && !EXACT) if (fast) {
+            RowCellD pd;
+            double mu[3];
+            row_cell_d<MODE>(a, c, valid, pd, mu);
+            const double xb = pd.beta * mu[0], xs = pd.beta * mu[1], xq = pd.beta * mu[2];
+            for (int q = -1; q <= 1; q++) fug[fug_row_d(0, q) * kT] = exp(q * xb);
+            for (int q = -3; q <= 3; q++) fug[fug_row_d(1, q) * kT] = exp(q * xs);
+            for (int q = -2; q <= 2; q++) fug[fug_row_d(2, q) * kT] = exp(q * xq);
+            const double* dnq_row = (a.dnq && valid) ? a.dnq + c * Ns : nullptr;
+            const double* kt = reinterpret_cast<const double*>(s_k);
+            const char* fcol = reinterpret_cast<const char*>(fug);
+#pragma unroll 1
+            for (int s = sbeg; s < min(nslow, send); s++) {
+                const RowSpD& q = rowsp[s];
+                double y = s < L ? row_yield_d<MODE, kLightTerms>(q, pd, fcol, kt)
+                                 : row_yield_d<MODE, 1>(q, pd, fcol, kt);
+                if (dnq_row && s < Ns && q.g != 0.) y += dnq_row[s];
+                y = fmax(y, 0.);
+                if (valid) row[s] = y;
+                ctot += y;
+                const double t = wave_sum_dpp(y);
+                if (lane == 0) wacc[s] += t;
+            }
+#pragma unroll 1
+            for (int s0 = max(sbeg, nslow); s0 < send; s0 += SC) {
+                double y[SC];
+#pragma unroll
+                for (int j = 0; j < SC; j++) y[j] = row_yield_d<MODE, 1>(rowsp[s0 + j], pd, fcol, kt);
+                if (dnq_row) {
+#pragma unroll
+                    for (int j = 0; j < SC; j++)
+                        if (s0 + j < Ns && rowsp[s0 + j].g != 0.) y[j] += dnq_row[s0 + j];
+                }
+#pragma unroll
+                for (int j = 0; j < SC; j++) {
+                    y[j] = fmax(y[j], 0.);
+                    ctot += y[j];
+                }
+                if (valid) {
+#pragma unroll
+                    for (int k = 0; k < SC; k += 2)
+                        *reinterpret_cast<double2*>(row + s0 + k) = make_double2(y[k], y[k + 1]);
+                }
+                const double t = wave_sum8(y);
+                if ((lane & 7) == 0) wacc[s0 + wave_sum8_index(lane)] += t;
+            }
+            if (__any(valid && !rows_inside(a, pd.T, pd.beta)) && lane == 0) *a.oob = 1;
+        }
         if (!fast) one_by_one();
-        if (valid && a.ctot) a.ctot[c] = ctot;
+        if (valid && a.ctot) {
+            if (a.ctot_part) a.ctot_part[(wid - wk.owner(tile * tcost)) * Nc + c] = ctot;
+            else a.ctot[c] = ctot;
+        }
     }
     __syncthreads();
     for (int s = threadIdx.x; s < Ns; s += blockDim.x) {
         double t = 0.;
-        for (int k = 0; k < kRowThreads / kWave; k++) t += s_acc[k * stride + s];
+        for (int k = 0; k < kT / kWave; k++) t += s_acc[k * stride + s];
         a.partial[static_cast<int64_t>(blockIdx.x) * Ns + s] = t;
     }
 }
