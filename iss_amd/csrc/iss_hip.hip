@@ -897,14 +897,13 @@ int mlp_step(iss_ctx* ctx, TrainArgs& t, int nb, float lr, float* grad_out) {
     t.loss_part = ctx->d_tloss.p;
     HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mlp_train),
                                hipFuncAttributeMaxDynamicSharedMemorySize, kTrainLds));
-    k_mlp_train<<<nb, 64, kTrainLds, ctx->stream>>>(t);
+    k_mlp_train<<<nb, kTrainThreads, kTrainLds, ctx->stream>>>(t);
     HIPCHK(hipGetLastError());
     if (lr > 0.f) ctx->adam_t++;
-    k_mlp_reduce_adam<<<(kNumParams + 255) / 256, 256, 0, ctx->stream>>>(
-        ctx->d_tpart.p, nb, ctx->d_tloss.p, ctx->d_mlp_par.p, ctx->d_adam_m.p, ctx->d_adam_v.p, grad_out, lr,
-        ctx->adam_t);
+    k_mlp_reduce_adam<<<(kNumParams + 63) / 64, 64, 0, ctx->stream>>>(
+        ctx->d_tpart.p, nb, ctx->d_tloss.p, ctx->d_mlp_par.p, ctx->d_adam_m.p, ctx->d_adam_v.p, grad_out,
+        ctx->d_mlp_frag.p, lr, ctx->adam_t);
     HIPCHK(hipGetLastError());
-    if (lr > 0.f) return mlp_pack(ctx);
     return ISS_OK;
 }
 
