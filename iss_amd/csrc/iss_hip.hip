@@ -340,7 +340,9 @@ struct iss_ctx {
     double k_first = 0., k_last = 0., k_light = 0.;  // range of the row pass's K arguments (YieldArgs)
     bool light_beyond = false;  // a species below 0.7 GeV after the first nlight ones
     DBuf<char> d_rows;
-    DBuf<float4> d_ecell;      // [2 Nc]: per cell flow and 3+1D position (k_emit_cells)
+    DBuf<float4> d_tcell;      // [Nc][kTCell]: the trial kernels' cell words (k_trial_cells), built by the
+    bool tcell_ready = false;  // first sampling pass of a surface and delta f
+    DBuf<TSpec> d_tspec;
     DBuf<RowSp> d_rowsp;       // [2][row_stride(Ns, 4)]: all species, then negative charges suppressed
     bool charges_outside = false;  // a species charge beyond the row pass's fugacity rows
     DBuf<RowSpD> d_rowspd;     // the same in FP64, [2][row_stride(Ns, 8)]
@@ -526,10 +528,20 @@ int build_ptables(iss_ctx* ctx, int quirk) {
             r[2] = host_pcdf(fer, quirk, tr[t], m0s[t], 2, e);
         }
     }
+    // tables 0 and 3 once more as the trial kernel stages them: three entries
+    // a row, zero beyond the table
+    const size_t rows = h.size();
+    h.resize(rows + 2ull * kPTabLen * 3, 0.);
+    for (int t = 0; t < 2; t++)
+        for (int i = 0; i < kPTabLen; i++)
+            for (int k = 0; k < 3; k++)
+                h[rows + (static_cast<size_t>(t) * kPTabLen + i) * 3 + k] =
+                    h[(static_cast<size_t>(3 * t) * kPTabLen + i) * 4 + k];
     HIPCHK(ctx->d_ptab.ensure(h.size()));
     HIPCHK(hipMemcpyAsync(ctx->d_ptab.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice,
                           ctx->stream));
     pt.C = ctx->d_ptab.p;
+    pt.packed = ctx->d_ptab.p + rows;
     return ISS_OK;
 }
 
@@ -581,12 +593,31 @@ int cell_prep(iss_ctx* ctx) {
         HIPCHK(ctx->d_aux.ensure(static_cast<size_t>(kAuxFields) * ctx->Nc));
         k_cell_aux<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_aux.p);
         HIPCHK(hipGetLastError());
-        HIPCHK(ctx->d_ecell.ensure(2 * ctx->Nc));
-        k_emit_cells<<<nb, 256, 0, ctx->stream>>>(ctx->d_cells.p, ctx->Nc, ctx->d_ecell.p);
-        HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    ctx->tcell_ready = false;
     return ISS_OK;
+}
+
+// the trial kernels' cell words, by the first sampling pass of a surface and
+// delta f (yields and spectra need none)
+int ensure_tcell(iss_ctx* ctx) {
+    if (ctx->tcell_ready || ctx->Nc <= 0) return ISS_OK;
+    HIPCHK(ctx->d_tcell.ensure(static_cast<size_t>(kTCell) * ctx->Nc));
+    k_trial_cells<<<(ctx->Nc + 255) / 256, 256, 0, ctx->stream>>>(
+        ctx->d_cells.p, ctx->d_coef.p, ctx->Nc, ctx->df.include_bulk && ctx->bulk_mode == BULK_RTA,
+        ctx->df.include_diffusion, ctx->d_tcell.p);
+    HIPCHK(hipGetLastError());
+    ctx->tcell_ready = true;
+    return ISS_OK;
+}
+
+// blocks of a plain trial launch over K hadrons: one per 64 hadrons, at most
+// the resident ones, so that few hadrons spread over the CUs (a pass ends
+// with its longest chain of trials, whose iterations a full CU slows)
+int trial_blocks(const iss_ctx* ctx, int64_t K, int per_cu) {
+    return static_cast<int>(
+        std::max<int64_t>(1, std::min<int64_t>((K + kWave - 1) / kWave, int64_t(ctx->num_cu) * per_cu)));
 }
 
 SpeciesDev species_dev(iss_ctx* ctx) {
@@ -1117,7 +1148,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_ctot.release(); ctx->d_ctot_part.release(); ctx->d_rowspd.release(); ctx->d_partial.release(); ctx->d_oob.release(); ctx->d_stot.release(); ctx->d_raw.release();
     ctx->d_counts.release(); ctx->d_evcount.release(); ctx->d_off.release(); ctx->d_evoff.release();
     ctx->d_tree0.release(); ctx->d_tree1.release(); ctx->d_out.release(); ctx->d_setup.release(); ctx->d_stats.release();
-    ctx->d_cellidx.release(); ctx->d_ecell.release();
+    ctx->d_cellidx.release(); ctx->d_tcell.release(); ctx->d_tspec.release();
     ctx->d_ycol.release(); ctx->d_mcnt.release(); ctx->d_msegoff.release(); ctx->d_msp.release();
     ctx->d_anti.release(); ctx->d_lcc_flag.release(); ctx->d_lcc_g.release(); ctx->d_lcc_src.release();
     ctx->d_lcc_evoff.release(); ctx->d_lcc_rec.release(); ctx->d_out2.release();
@@ -1191,6 +1222,11 @@ int iss_set_species(iss_ctx* ctx, const iss_species_desc* sp) {
     HIPCHK(hipMemcpyAsync(ctx->d_mass.p, sp->mass, sizeof(double) * Ns, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(ctx->d_ints.p, ints.data(), sizeof(int) * 6 * Ns, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(ctx->d_spk.p, spk.data(), sizeof(SpeciesK) * Ns, hipMemcpyHostToDevice, ctx->stream));
+    std::vector<TSpec> tsp(Ns);
+    for (int i = 0; i < Ns; i++)
+        tsp[i] = TSpec{sp->mass[i], spk[i].B, spk[i].S, spk[i].Q, spk[i].sgn, sp->pid[i], spk[i].m};
+    HIPCHK(ctx->d_tspec.ensure(Ns));
+    HIPCHK(hipMemcpyAsync(ctx->d_tspec.p, tsp.data(), sizeof(TSpec) * Ns, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->Ns = Ns;
     // the leading species below 0.7 GeV take the 10-term series (the row
@@ -1521,9 +1557,7 @@ static int lcc_partners(iss_ctx* ctx, const SampleArgs& a, int E, const HSetup* 
         ap.out = ctx->d_out2.p;
         ap.K = P;
         ap.Kdev = nullptr;
-        const int nblk = static_cast<int>(
-            std::max<int64_t>(1, std::min<int64_t>((P + kTrialThreads - 1) / kTrialThreads, int64_t(ctx->num_cu) * per_cu_plain)));
-        k_trials<<<nblk, kTrialThreads, 0, ctx->stream>>>(ap, ctx->d_lcc_rec.p);
+        k_trials<<<trial_blocks(ctx, P, per_cu_plain), kTrialThreads, 0, ctx->stream>>>(ap, ctx->d_lcc_rec.p);
         HIPCHK(hipGetLastError());
     }
     k_lcc_events<<<(E + 1 + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_evoff.p, E, ctx->d_lcc_g.p, ctx->d_lcc_evoff.p);
@@ -1577,6 +1611,8 @@ static int sample_model(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadro
     HIPCHK(hipGetLastError());
     rc = launch_scan(ctx, ctx->d_mcnt.p, nseg, ctx->d_msegoff.p);
     if (rc) return rc;
+    rc = ensure_tcell(ctx);
+    if (rc) return rc;
     k_model_evoff<<<(E + 1 + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_msegoff.p, E, Ns, ctx->d_evoff.p);
     int64_t K = 0;
     HIPCHK(hipMemcpyAsync(&K, ctx->d_msegoff.p + nseg, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -1594,7 +1630,8 @@ static int sample_model(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadro
     a.seed = o->seed;
     a.chunk = chunk;
     a.boost_invariant = binv ? 1 : 0;
-    a.ecell = binv ? nullptr : ctx->d_ecell.p;  // 3+1D: the cells' flow and position words
+    a.tcell = ctx->d_tcell.p;
+    a.tspec = ctx->d_tspec.p;
     a.yLB = static_cast<float>(o->y_LB);
     a.yRB = static_cast<float>(o->y_RB);
     a.max_trials = o->max_trials;
@@ -1613,9 +1650,7 @@ static int sample_model(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadro
         per_cu = 1;
     if (ctx->blocks_per_cu[0] > 0) per_cu = std::min(ctx->blocks_per_cu[0], per_cu);
     if (K > 0) {
-        const int nblk = static_cast<int>(std::max<int64_t>(
-            1, std::min<int64_t>((K + kTrialThreads - 1) / kTrialThreads, int64_t(ctx->num_cu) * per_cu)));
-        k_trials<<<nblk, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
+        k_trials<<<trial_blocks(ctx, K, per_cu), kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
         HIPCHK(hipGetLastError());
     }
     ctx->last_plain = true;  // the records' output slots index d_out
@@ -1714,6 +1749,8 @@ int iss_sample(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadrons) {
     HIPCHK(hipGetLastError());
     rc = launch_scan(ctx, ctx->d_evcount.p, E, ctx->d_evoff.p);
     if (rc) return rc;
+    rc = ensure_tcell(ctx);
+    if (rc) return rc;
     HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * ctx->Ns));
     HIPCHK(hipMemcpyAsync(ctx->h_pin.at<int64_t>(PIN_K), ctx->d_off.p + Nc, sizeof(int64_t), hipMemcpyDeviceToHost,
                           ctx->stream));
@@ -1741,7 +1778,8 @@ int iss_sample(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadrons) {
     a.neos = ctx->neos;
     a.diff = ctx->df.include_diffusion;
     a.boost_invariant = binv ? 1 : 0;
-    a.ecell = binv ? nullptr : ctx->d_ecell.p;  // 3+1D: the cells' flow and position words
+    a.tcell = ctx->d_tcell.p;
+    a.tspec = ctx->d_tspec.p;
     a.yLB = static_cast<float>(o->y_LB);
     a.yRB = static_cast<float>(o->y_RB);
     a.max_trials = o->max_trials;
@@ -1796,10 +1834,7 @@ int iss_sample(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadrons) {
             HIPCHK(hipEventRecord(ctx->ev[7], ctx->stream));
             k_setup<false><<<(K + 255) / 256, 256, 0, ctx->stream>>>(a, ctx->d_setup.p, nullptr, nullptr);
             HIPCHK(hipEventRecord(ctx->ev[6], ctx->stream));
-            const int64_t want = (K + kTrialThreads - 1) / kTrialThreads;
-            const int nblk = static_cast<int>(
-                std::max<int64_t>(1, std::min<int64_t>(want, int64_t(ctx->num_cu) * per_cu_plain)));
-            k_trials<<<nblk, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
+            k_trials<<<trial_blocks(ctx, K, per_cu_plain), kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
         }
         ctx->last_plain = true;
     } else {
@@ -2364,6 +2399,10 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     HIPCHK(ctx->d_lam.ensure(S));
     HIPCHK(ctx->d_bevents.ensure(S));
     HIPCHK(hipMemcpyAsync(ctx->d_bevents.p, n_events, sizeof(int32_t) * S, hipMemcpyHostToDevice, ctx->stream));
+    {
+        const int rc = ensure_tcell(ctx);
+        if (rc) return rc;
+    }
     k_batch_lambda<<<S, 256, 0, ctx->stream>>>(ctx->d_surf_off.p, ctx->d_ctot.p, ctx->d_lam.p);
     HIPCHK(hipGetLastError());
     std::vector<double> lam(S);
@@ -2423,7 +2462,8 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     a.cellidx = ctx->d_cellidx.p;
     a.slot_species = ctx->d_sp16.p;  // (every slot's species from the round's pick)
     a.boost_invariant = binv ? 1 : 0;
-    a.ecell = binv ? nullptr : ctx->d_ecell.p;  // 3+1D: the cells' flow and position words
+    a.tcell = ctx->d_tcell.p;
+    a.tspec = ctx->d_tspec.p;
     a.yLB = static_cast<float>(o->y_LB);
     a.yRB = static_cast<float>(o->y_RB);
     a.max_trials = o->max_trials;
@@ -2435,7 +2475,7 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
         per_cu = 1;
     const int per_cu_fb = per_cu;  // (the learned rounds' plain fallback)
     if (ctx->blocks_per_cu[0] > 0) per_cu = std::min(ctx->blocks_per_cu[0], per_cu);
-    const int trial_blocks = ctx->num_cu * per_cu;
+    const int nblk_trials = ctx->num_cu * per_cu;
     const int setup_blocks = ctx->num_cu * 8;
     const int64_t ntiles = std::max<int64_t>(1, (N + kScanTile - 1) / kScanTile);
     // learned proposal: the round's (cell, species) pairs, one network
@@ -2519,7 +2559,7 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
         }
         if (!learned) {
             k_setup<true><<<setup_blocks, 256, 0, ctx->stream>>>(a, ctx->d_setup.p, nullptr, nullptr);
-            k_trials<<<trial_blocks, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
+            k_trials<<<nblk_trials, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
         } else {
             k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_lcnt.p, N, ctx->d_scan.p);
             k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(ctx->d_scan.p, ntiles);

@@ -9,7 +9,9 @@
 //   ctot    double [Nc]               per-cell total yield (last cdf entry)
 //   ktab    double [3][kKLen]         K1, K2, K3 at x = 0.5 + 0.05 i
 //   ktabf   float2 [3][kKLen]         (K_i, K_{i+1} - K_i) for the FP32 pass
-//   ptab    double [6][3][2001]       |p|-sampler CDF_0/1/2 tables
+//   ptab    double [6][2001][4]       |p|-sampler CDF_0/1/2 tables, then tables 0
+//                                     and 3 as [2][2001][3]
+//   tcell   float4 [Nc][10]           the trial kernels' words of a cell
 #pragma once
 
 #include "device.h"
@@ -116,7 +118,8 @@ struct PTabDev {
     double ep[6], em1[6];  // exp(m0), exp(-m0)
     int len[6], trunc[6], fermion[6];
     int quirk;
-    const double* C;  // [6][3][kPTabLen]
+    const double* C;  // [6][kPTabLen][4]
+    const double* packed;  // [2][kPTabLen][3]: tables 0 and 3 as the trial kernel stages them
 };
 
 struct YieldArgs {
@@ -193,11 +196,34 @@ struct SampleArgs {
     const uint32_t* cellidx;
     // the species of every slot (k_pick); null: drawn from the FP64 species CDF rows
     const uint16_t* slot_species;
-    // 3+1D surfaces: per cell (u0, u1, u2, u3) and (t, x, y, z) (k_emit_cells),
-    // loaded when a trial lane takes a hadron; null: emit_lab gathers them
-    const float4* ecell;
+    // per-cell and per-species words of the trial kernels (k_trial_cells,
+    // TSpec), loaded when a trial lane takes a hadron
+    const float4* tcell;
+    const struct TSpec* tspec;
 };
 
 constexpr uint32_t kPartnerBit = 0x80000000u;
+
+// what a trial lane needs of its cell, as kTCell 16-byte words
+enum TCellWord {
+    TC_T = 0,    // T, mu_B, mu_S, mu_Q
+    TC_DS,       // dsigma_mu
+    TC_PRE,      // 1 / (|ds0| + |ds|), 1 / T, 1 / (2 T^2 (e + P)), Pi (over hbar c for the RTA)
+    TC_PI,       // pi_xx, pi_xy, pi_xz, pi_yy
+    TC_PC,       // pi_yz, bulk / NEoS coefficients 0, 1, 2
+    TC_C,        // coefficients 3, 4, 5, n_B / (e + P)
+    TC_Q,        // q / D_qmu, -
+    TC_U, TC_X,  // flow u; 3+1D position (t, x, y, z)
+    TC_B,        // 1 / T in FP64 (two words), -, -
+    kTCell
+};
+// ... and of its species
+struct alignas(16) TSpec {
+    double mass;
+    float B, S, Q, sgn;
+    int pid;
+    float fm;
+};
+static_assert(sizeof(TSpec) == 32, "TSpec is two 16-byte words");
 
 }  // namespace issdev

@@ -1129,9 +1129,9 @@ __global__ __launch_bounds__(256) void k_learn_trials(LearnArgs L, const LRec* _
             const float px = p * (R00 * n0 + R01 * n1 + R02 * n2);
             const float py = p * (R10 * n0 + R11 * n1 + R12 * n2);
             const float pz = p * (R20 * n0 + R21 * n1 + R22 * n2);
-            if (a.ecell) {
-                const float4* ec = a.ecell + 2 * static_cast<int64_t>(c);
-                emit_cell_lab(a, ec[0], ec[1], a.sp.pid[s], P.m, px, py, pz, E, outp);
+            if (!a.boost_invariant) {
+                const float4* tc = a.tcell + static_cast<int64_t>(c) * kTCell;
+                emit_cell_lab(a, tc[TC_U], tc[TC_X], a.sp.pid[s], P.m, px, py, pz, E, outp);
             }
             else emit_lab(a, chunk, c, jj, a.sp.pid[s], P.m, px, py, pz, E, outp);
             done = true;

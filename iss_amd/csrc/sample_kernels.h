@@ -225,19 +225,46 @@ __device__ __forceinline__ void emit_lab(const SampleArgs& a, uint32_t chunk, in
     static_cast<Hadron*>(a.out)[outp] = h;
 }
 
-// The per-cell part of the lab-frame record on 3+1D surfaces: the flow and
-// the position (t, x, y, z) = (tau cosh eta, x, y, tau sinh eta), once per
-// surface with the operations of emit_lab, so that a trial lane loads two
-// 16-byte words when it takes a hadron instead of gathering eight fields
-// (and evaluating cosh and sinh) at every acceptance.
-__global__ void k_emit_cells(const float* __restrict__ cells, int64_t Nc, float4* __restrict__ ec) {
-    for (int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; c < Nc;
-         c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const float tau = cells[F_TAU * Nc + c], eta = cells[F_ETA * Nc + c];
-        ec[2 * c] = make_float4(cells[F_U0 * Nc + c], cells[F_U1 * Nc + c], cells[F_U2 * Nc + c],
-                                cells[F_U3 * Nc + c]);
-        ec[2 * c + 1] = make_float4(tau * coshf(eta), cells[F_X * Nc + c], cells[F_Y * Nc + c], tau * sinhf(eta));
+// The per-cell words of the trial kernels, once per surface and delta f: a
+// lane that takes a hadron loads ten 16-byte words of one record instead of
+// gathering some thirty fields from as many arrays, and what depends on the
+// cell alone (square root, reciprocals, the position (t, x, y, z) = (tau cosh
+// eta, x, y, tau sinh eta) of emit_lab on 3+1D surfaces) is not recomputed
+// per hadron.  The operations are those of the per-hadron forms.
+__global__ void k_trial_cells(const float* __restrict__ cells, const double* __restrict__ coef, int64_t Nc,
+                              int rta, int diff, float4* __restrict__ tc) {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (c >= Nc) return;
+    auto F = [&](int f) { return cells[f * Nc + c]; };
+    float4* w = tc + c * kTCell;
+    const float T = F(F_T), Ed = F(F_E), Pd = F(F_P);
+    const float d0 = F(F_DA0), d1 = F(F_DA1), d2 = F(F_DA2), d3 = F(F_DA3);
+    const float dsfac = fabsf(d0) + sqrtf(d1 * d1 + d2 * d2 + d3 * d3);
+    float Pi = F(F_PI);
+    if (rta) Pi = Pi / static_cast<float>(kHbarC);
+    float cf[6];
+    for (int k = 0; k < 6; k++) cf[k] = coef[k * Nc + c];
+    float q[3] = {0.f, 0.f, 0.f}, pqm = 0.f;
+    if (diff) {
+        const float iq = static_cast<float>(coef[6 * Nc + c]);
+        q[0] = F(F_QX) * iq;
+        q[1] = F(F_QY) * iq;
+        q[2] = F(F_QZ) * iq;
+        pqm = static_cast<float>(coef[7 * Nc + c]);
     }
+    const float tau = F(F_TAU), eta = F(F_ETA);
+    const uint64_t beta = __builtin_bit_cast(uint64_t, 1. / static_cast<double>(T));
+    w[TC_T] = make_float4(T, F(F_MUB), F(F_MUS), F(F_MUQ));
+    w[TC_DS] = make_float4(d0, d1, d2, d3);
+    w[TC_PRE] = make_float4(1.0f / dsfac, 1.0f / T, 1.0f / (2.0f * T * T * (Ed + Pd)), Pi);
+    w[TC_PI] = make_float4(F(F_PIXX), F(F_PIXY), F(F_PIXZ), F(F_PIYY));
+    w[TC_PC] = make_float4(F(F_PIYZ), cf[0], cf[1], cf[2]);
+    w[TC_C] = make_float4(cf[3], cf[4], cf[5], pqm);
+    w[TC_Q] = make_float4(q[0], q[1], q[2], 0.f);
+    w[TC_U] = make_float4(F(F_U0), F(F_U1), F(F_U2), F(F_U3));
+    w[TC_X] = make_float4(tau * coshf(eta), F(F_X), F(F_Y), tau * sinhf(eta));
+    w[TC_B] = make_float4(__uint_as_float(static_cast<uint32_t>(beta)), __uint_as_float(static_cast<uint32_t>(beta >> 32)),
+                          0.f, 0.f);
 }
 
 // emit_lab on a 3+1D surface from the cell's words eu = u, ep = (t, x, y, z):
@@ -337,6 +364,31 @@ __device__ __forceinline__ void pstate_of(const SampleArgs& a, int64_t c, int s,
     q.fsg = static_cast<float>(a.sp.sign[s]);
 }
 
+// n / d, correctly rounded, from the correctly rounded reciprocal r of d (two
+// residual corrections, P. Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", IBM J. Res. Dev. 34 (1990) 111-119)
+__device__ __forceinline__ double div_by(double n, double d, double r) {
+    const double q0 = n * r;
+    const double q1 = fma(fma(-q0, d, n), r, q0);
+    return fma(fma(-q1, d, n), r, q1);
+}
+
+// pstate_of from the trial words of the cell and species: the divisions by T
+// through the cell's 1 / T, with the same results
+__device__ __forceinline__ void pstate_cell(const float4& wT, const float4& wB, const TSpec& sp, PState& q) {
+    q.T = wT.x;
+    q.mu = fmin(sp.mass, static_cast<double>(sp.B * wT.y + sp.S * wT.z + sp.Q * wT.w));
+    q.Td = q.T;
+    const double beta = __builtin_bit_cast(
+        double, (static_cast<uint64_t>(__float_as_uint(wB.y)) << 32) | __float_as_uint(wB.x));
+    const double mt = div_by(sp.mass, q.Td, beta);
+    q.mut = div_by(q.mu, q.Td, beta);
+    q.x = mt - q.mut;
+    q.aa = q.mut * q.mut - mt * mt / 2.;
+    q.fm = sp.fm;
+    q.fmu = static_cast<float>(q.mu);
+    q.fsg = sp.sgn;
+}
 
 // Species of every hadron slot of a pass, one wave per cell.  By Poisson
 // splitting a hadron of cell c is of species s with probability
@@ -513,9 +565,9 @@ __device__ __forceinline__ uint64_t batch_out(const SampleArgs& a, int64_t i, in
 // row and the proposal's normalisation at E~ = m~ - mu~
 __device__ __forceinline__ HSetup setup_record(const SampleArgs& a, int64_t c, uint32_t jj, int s) {
     PState q;
-    pstate_of(a, c, s, q);
-    const int sign = a.sp.sign[s];
-    const int tb = ((sign == -1) ? 0 : 3) + ((q.x < 30.) ? 0 : (q.x < 50. ? 1 : 2));
+    const float4* tc = a.tcell + c * kTCell;
+    pstate_cell(tc[TC_T], tc[TC_B], a.tspec[s], q);
+    const int tb = ((q.fsg == -1.f) ? 0 : 3) + ((q.x < 30.) ? 0 : (q.x < 50. ? 1 : 2));
     double cm[3];
     pcdf_all(a.pt, tb, q.x, cm);
     HSetup r;
@@ -588,21 +640,26 @@ constexpr int kRefillMin = 16;
 // nearly every hadron uses, are copied into LDS (e0, e1, e2 per row, 96 KB)
 // by each workgroup, one workgroup of kTrialThreads per CU (4 waves per SIMD
 // at the kernel's registers): the bracket search runs in LDS, without
-// dependent global loads.  (The search over LDS rows g kCoarse narrows the
-// bracket; with every row there, kCoarse = 1, it finds it.)  Other tables
-// are searched in global memory.
+// dependent global loads.  Other tables are searched in global memory.
+// What bounds it at 9.5M hadrons: vector issue (about 570 instructions an
+// iteration) and the waits of its two chains, the refill's loads and the
+// search's dependent LDS reads.  964 -> 840 us from one record per cell
+// instead of gathers, the search's rows read together, 64-bit Philox
+// products and the tables staged by 16-byte copies.
 constexpr int kTrialThreads = 1024;
-constexpr int kCoarse = 1;
-constexpr int kCoarseRows = (kPTabLen + kCoarse - 1) / kCoarse;
 
 __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* __restrict__ rec) {
     __shared__ unsigned long long s_stats[4];
-    __shared__ double s_ctab[2][kCoarseRows * 3];
+    __shared__ __align__(16) double s_ctab[2 * kPTabLen * 3];
     if (threadIdx.x < 4) s_stats[threadIdx.x] = 0ull;
-    for (int i = threadIdx.x; i < 2 * kCoarseRows * 3; i += blockDim.x) {
-        const int t = i / (kCoarseRows * 3), g = (i / 3) % kCoarseRows, k = i % 3;
-        const int tbl = t == 0 ? 0 : 3, row = g * kCoarse;
-        s_ctab[t][g * 3 + k] = row < a.pt.len[tbl] ? a.pt.C[(static_cast<int64_t>(tbl) * kPTabLen + row) * 4 + k] : 0.;
+    {
+        const double2* src = reinterpret_cast<const double2*>(a.pt.packed);
+        double2* dst = reinterpret_cast<double2*>(s_ctab);
+#pragma unroll
+        for (int k = 0; k < (kPTabLen * 3 + kTrialThreads - 1) / kTrialThreads; k++) {
+            const int i = k * kTrialThreads + threadIdx.x;
+            if (i < kPTabLen * 3) dst[i] = src[i];
+        }
     }
     __syncthreads();
     const int lane = threadIdx.x & (kWave - 1);
@@ -614,7 +671,6 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
     const int64_t base = Kn / nwaves, rem = Kn % nwaves;
     const int64_t beg = wid * base + min(wid, rem);
     const int64_t end = beg + base + (wid < rem ? 1 : 0);
-    const int64_t Nc = a.Nc;
     const PTabDev& pt = a.pt;
     const uint32_t key0 = static_cast<uint32_t>(a.seed), key1 = static_cast<uint32_t>(a.seed >> 32);
     const uint32_t tw = tag_word(TAG_TRIAL, chunk);
@@ -629,9 +685,9 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
     uint64_t outp = 0;
     uint32_t jj = 0;
     int s = 0, tb = 0, i0 = 0, imax = 0, it = 0, trials = 1;
-    double mterm = 0., cmax = 0., rmin0 = 0.;
+    double mterm = 0., cmax = 0.;
     PState q{};
-    float dsfac = 1.f, rdsfac = 1.f, rT = 1.f, dfpref = 0.f, d0 = 0.f, d1 = 0.f, d2 = 0.f, d3 = 0.f, Pi = 0.f;
+    float rdsfac = 1.f, rT = 1.f, dfpref = 0.f, d0 = 0.f, d1 = 0.f, d2 = 0.f, d3 = 0.f, Pi = 0.f;
     float Bq = 0.f, Sq = 0.f, Qq = 0.f;
     float pixx = 0.f, pixy = 0.f, pixz = 0.f, piyy = 0.f, piyz = 0.f;
     float cf0 = 0.f, cf1 = 0.f, cf2 = 0.f, cf3 = 0.f, cf4 = 0.f, cf5 = 0.f;
@@ -653,40 +709,28 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
                 i0 = r.i0;
                 mterm = r.mterm;
                 outp = r.out;
-                pstate_of(a, c, s, q);
-                if (a.ecell) {
-                    eu = a.ecell[2 * c];
-                    ep = a.ecell[2 * c + 1];
-                    pid = a.sp.pid[s];
+                const float4* tc = a.tcell + c * kTCell;
+                const float4 wT = tc[TC_T], wD = tc[TC_DS], wP = tc[TC_PRE], wB = tc[TC_B];
+                const TSpec sp = a.tspec[s];
+                if (!a.boost_invariant) {
+                    eu = tc[TC_U];
+                    ep = tc[TC_X];
                 }
-                d0 = a.cells[F_DA0 * Nc + c]; d1 = a.cells[F_DA1 * Nc + c];
-                d2 = a.cells[F_DA2 * Nc + c]; d3 = a.cells[F_DA3 * Nc + c];
-                const float Ed = a.cells[F_E * Nc + c], Pd = a.cells[F_P * Nc + c];
-                Bq = a.sp.B[s]; Sq = a.sp.S[s]; Qq = a.sp.Q[s];
-                dsfac = fabsf(d0) + sqrtf(d1 * d1 + d2 * d2 + d3 * d3);
-                rdsfac = 1.0f / dsfac;
-                rT = 1.0f / q.T;
-                dfpref = 1.0f / (2.0f * q.T * q.T * (Ed + Pd));
-                if (a.shear) {
-                    pixx = a.cells[F_PIXX * Nc + c]; pixy = a.cells[F_PIXY * Nc + c];
-                    pixz = a.cells[F_PIXZ * Nc + c]; piyy = a.cells[F_PIYY * Nc + c];
-                    piyz = a.cells[F_PIYZ * Nc + c];
-                }
-                if (a.bulk != BULK_NONE) {
-                    Pi = a.cells[F_PI * Nc + c];
-                    if (a.bulk == BULK_RTA) Pi = Pi / static_cast<float>(kHbarC);
-                }
-                if (a.bulk != BULK_NONE || a.neos >= 0) {
-                    cf0 = a.coef[c]; cf1 = a.coef[Nc + c]; cf2 = a.coef[2 * Nc + c];
-                    cf3 = a.coef[3 * Nc + c]; cf4 = a.coef[4 * Nc + c]; cf5 = a.coef[5 * Nc + c];
+                if (a.shear || a.bulk != BULK_NONE || a.neos >= 0) {
+                    const float4 w0 = tc[TC_PI], w1 = tc[TC_PC], w2 = tc[TC_C];
+                    pixx = w0.x; pixy = w0.y; pixz = w0.z; piyy = w0.w; piyz = w1.x;
+                    cf0 = w1.y; cf1 = w1.z; cf2 = w1.w; cf3 = w2.x; cf4 = w2.y; cf5 = w2.z;
                 }
                 if (a.diff) {
-                    const float iq = static_cast<float>(a.coef[6 * Nc + c]);
-                    qx = a.cells[F_QX * Nc + c] * iq;
-                    qy = a.cells[F_QY * Nc + c] * iq;
-                    qz = a.cells[F_QZ * Nc + c] * iq;
-                    pqm = static_cast<float>(a.coef[7 * Nc + c]);
+                    const float4 wq = tc[TC_Q];
+                    qx = wq.x; qy = wq.y; qz = wq.z;
+                    pqm = tc[TC_C].w;
                 }
+                d0 = wD.x; d1 = wD.y; d2 = wD.z; d3 = wD.w;
+                rdsfac = wP.x; rT = wP.y; dfpref = wP.z; Pi = wP.w;
+                Bq = sp.B; Sq = sp.S; Qq = sp.Q;
+                pid = sp.pid;
+                pstate_cell(wT, wB, sp, q);
                 it = 0;
                 trials = 1;
                 imax = pt.len[tb] - 1;
@@ -696,9 +740,7 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
                     n_range++;
                     write_hole(a, outp);
                 } else {
-                    const double* e0 = pt.C + (static_cast<int64_t>(tb) * kPTabLen + i0) * 4;
                     const double* em = pt.C + (static_cast<int64_t>(tb) * kPTabLen + imax) * 4;
-                    rmin0 = e0[2] + 2. * q.mut * e0[1] + q.aa * e0[0] - mterm;
                     cmax = em[2] + 2. * q.mut * em[1] + q.aa * em[0] - mterm;
                     active = true;
                 }
@@ -714,59 +756,45 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
         const u32x4 w = philox4x32(u32x4{static_cast<uint32_t>(c), jj, tw, static_cast<uint32_t>(it)}, key0, key1);
         it++;
         n_inner++;
-        const double* C = pt.C + static_cast<int64_t>(tb) * kPTabLen * 4;
         const double r = u32d(w.x) * cmax;
         // the bracket comb(lo) <= r < comb(hi = lo + 1) is unique, so any
         // search reproduces the reference's bisection (inverse_CDF); a 4-ary
-        // search issues its three loads together
+        // search with its three rows read together and chosen by selects (as
+        // branches, the lanes' different paths read them one after the other)
         int lo = i0, hi = imax;
-        double rlo = rmin0, rhi = cmax;
-        auto comb_of = [&](double e0, double e1, double e2) { return e2 + 2. * q.mut * e1 + q.aa * e0 - mterm; };
-        auto comb = [&](int qq) {
-            const double* e = C + 4 * qq;
-            return comb_of(e[0], e[1], e[2]);
+        double rlo, rhi;
+        auto search = [&](auto comb) {
+            while (hi - lo > 4) {
+                const int qd = (hi - lo) >> 2;
+                const int m1 = lo + qd, m2 = lo + 2 * qd, m3 = lo + 3 * qd;
+                const double v1 = comb(m1), v2 = comb(m2), v3 = comb(m3);
+                const bool b1 = r < v1, b2 = r < v2, b3 = r < v3;
+                const int nl = b2 ? (b1 ? lo : m1) : (b3 ? m2 : m3);
+                hi = b2 ? (b1 ? m1 : m2) : (b3 ? m3 : hi);
+                lo = nl;
+            }
+            while (hi - lo > 1) {
+                const int mid = (hi + lo) >> 1;
+                const bool b = r < comb(mid);
+                hi = b ? mid : hi;
+                lo = b ? lo : mid;
+            }
+            rlo = comb(lo);
+            rhi = comb(hi);
         };
+        auto comb_of = [&](double e0, double e1, double e2) { return e2 + 2. * q.mut * e1 + q.aa * e0 - mterm; };
         if (tb == 0 || tb == 3) {
-            // LDS rows g kCoarse strictly inside (lo, hi): g in [ga, gb]; find
-            // L < H with comb(L kCoarse) <= r < comb(H kCoarse), L = ga - 1
-            // and H = gb + 1 standing for lo and hi
-            const double* Cc = s_ctab[tb == 0 ? 0 : 1];
-            auto combc = [&](int g) { return comb_of(Cc[3 * g], Cc[3 * g + 1], Cc[3 * g + 2]); };
-            const int ga = lo / kCoarse + 1, gb = (hi - 1) / kCoarse;
-            int L = ga - 1, H = gb + 1;
-            double vl = rlo, vh = rhi;
-            while (H - L > 4) {
-                const int qd = (H - L) >> 2;
-                const int m1 = L + qd, m2 = L + 2 * qd, m3 = L + 3 * qd;
-                const double v1 = combc(m1), v2 = combc(m2), v3 = combc(m3);
-                if (r < v2) {
-                    if (r < v1) { H = m1; vh = v1; } else { L = m1; vl = v1; H = m2; vh = v2; }
-                } else {
-                    if (r < v3) { L = m2; vl = v2; H = m3; vh = v3; } else { L = m3; vl = v3; }
-                }
-            }
-            while (H - L > 1) {
-                const int mid = (H + L) >> 1;
-                const double vm = combc(mid);
-                if (r < vm) { H = mid; vh = vm; } else { L = mid; vl = vm; }
-            }
-            if (L >= ga) { lo = L * kCoarse; rlo = vl; }
-            if (H <= gb) { hi = H * kCoarse; rhi = vh; }
-        }
-        while (hi - lo > 3) {
-            const int qd = (hi - lo) >> 2;
-            const int m1 = lo + qd, m2 = lo + 2 * qd, m3 = lo + 3 * qd;
-            const double v1 = comb(m1), v2 = comb(m2), v3 = comb(m3);
-            if (r < v2) {
-                if (r < v1) { hi = m1; rhi = v1; } else { lo = m1; rlo = v1; hi = m2; rhi = v2; }
-            } else {
-                if (r < v3) { lo = m2; rlo = v2; hi = m3; rhi = v3; } else { lo = m3; rlo = v3; }
-            }
-        }
-        while (hi - lo > 1) {
-            const int mid = (hi + lo) >> 1;
-            const double rm = comb(mid);
-            if (r < rm) { hi = mid; rhi = rm; } else { lo = mid; rlo = rm; }
+            const double* Cc = s_ctab + (tb == 0 ? 0 : kPTabLen * 3);
+            search([&](int g) {
+                const double* e = Cc + __umul24(g, 3);
+                return comb_of(e[0], e[1], e[2]);
+            });
+        } else {
+            const double* C = pt.C + static_cast<int64_t>(tb) * kPTabLen * 4;
+            search([&](int g) {
+                const double* e = C + 4 * g;
+                return comb_of(e[0], e[1], e[2]);
+            });
         }
         const double Et0 = pt.Et0[tb], dEt = pt.dEt[tb];
         double E0 = Et0 + lo * dEt;
@@ -821,8 +849,8 @@ __device__ __forceinline__ void trials_body(const SampleArgs& a, const HSetup* _
             const uint32_t u4 = (w.y & 0xFFu) | ((w.z & 0xFFu) << 8) | ((w.w & 0xFFu) << 16);
             const float ua = (static_cast<float>(u4) + 0.5f) * (1.0f / 16777216.0f);
             if (ua < w1 * w2) {
-                if (a.ecell) emit_cell_lab(a, eu, ep, pid, fm, px, py, pz, p0, outp);
-                else emit_lab(a, chunk, c, jj, a.sp.pid[s], fm, px, py, pz, p0, outp);
+                if (!a.boost_invariant) emit_cell_lab(a, eu, ep, pid, fm, px, py, pz, p0, outp);
+                else emit_lab(a, chunk, c, jj, pid, fm, px, py, pz, p0, outp);
                 done = true;
             } else {
                 trials++;
