@@ -281,7 +281,7 @@ __device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcn
 // and row_bcast:31 (0x143) pass lane 15 of each row, and lane 31, to the
 // following rows.  Lanes without a source, and rows outside row_mask, take
 // `old`.
-constexpr int kDppRowShr = 0x110, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
+constexpr int kDppRowShr = 0x110, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143, kDppWaveShr1 = 0x138;
 
 template <int CTRL, int ROW_MASK = 0xf>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t old, uint32_t v) {
@@ -317,6 +317,15 @@ __device__ __forceinline__ double wave_last(double v) {
     return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 // the sum over all lanes, returned uniformly (from lane 63 of the scan)
+// a 64-bit value of one lane (wave-uniform index), returned uniformly
+template <typename T>
+__device__ __forceinline__ T readlane64(T v, int l) {
+    static_assert(sizeof(T) == 8, "64-bit values");
+    const uint64_t x = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(x), l);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(x >> 32), l);
+    return __builtin_bit_cast(T, (static_cast<uint64_t>(hi) << 32) | lo);
+}
 __device__ __forceinline__ double wave_sum_dpp(double v) { return wave_last(wave_scan_dpp(v)); }
 // Running maximum over the lanes up to this one, in the steps of
 // wave_scan_dpp; for non-negative values (lanes without a source take 0)

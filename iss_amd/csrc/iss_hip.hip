@@ -612,6 +612,39 @@ int ensure_tcell(iss_ctx* ctx) {
     return ISS_OK;
 }
 
+// the species and cell of every slot of a pass (at most `slots`) from the
+// yield rows; the learned passes (bits) also get the pair bitmaps and counts.
+// Sparse passes take k_pick_few: rounds of 1.8e5 slots on some 4e5 cells
+// 102 -> 43 us, the densest (1.3 slots a cell) 186 -> 101.  Its serial slots
+// lose where cells hold many (50 a cell: 201 us against 144), and its waves
+// of 16 cells leave a small surface's chip idle.
+template <typename R>
+void launch_pick_t(iss_ctx* ctx, const SampleArgs& a, bool few, uint32_t* bits, uint32_t* cnt, uint32_t* scnt) {
+    const R* rows = reinterpret_cast<const R*>(ctx->d_rows.p);
+    const int stride = row_stride(ctx->Ns, sizeof(R));
+    if (few) {
+        // one instance per species a lane holds (1 to 8 of at most 512)
+        using Kernel = decltype(&k_pick_few<R, 1>);
+        static const Kernel kernels[8] = {k_pick_few<R, 1>, k_pick_few<R, 2>, k_pick_few<R, 3>, k_pick_few<R, 4>,
+                                          k_pick_few<R, 5>, k_pick_few<R, 6>, k_pick_few<R, 7>, k_pick_few<R, 8>};
+        const int blk = static_cast<int>((a.Nc + kPickCells * kPickSpan - 1) / (kPickCells * kPickSpan));
+        kernels[(ctx->Ns + kWave - 1) / kWave - 1]<<<blk, kWave * kPickCells, 0, ctx->stream>>>(
+            a.off, a.Nc, a.Ns, a.seed, a.chunk, a.chunk_dev, a.setup_cap, rows, stride, ctx->d_sp16.p, ctx->d_cellidx.p);
+        return;
+    }
+    const int blk = static_cast<int>((a.Nc + kPickCells - 1) / kPickCells);
+    const size_t lds = pick_lds_bytes(ctx->Ns, bits != nullptr);
+    auto kernel = bits ? k_pick<R, true> : k_pick<R, false>;
+    kernel<<<blk, kWave * kPickCells, lds, ctx->stream>>>(a, rows, stride, ctx->d_sp16.p, ctx->d_cellidx.p, bits, cnt,
+                                                          scnt, ctx->learn_route);
+}
+
+void launch_pick(iss_ctx* ctx, const SampleArgs& a, int64_t slots, uint32_t* bits, uint32_t* cnt, uint32_t* scnt) {
+    const bool few = !bits && slots <= 2 * a.Nc && a.Nc >= int64_t(kPickSpan) * 32 * ctx->num_cu;
+    if (ctx->yield_precision == 64) launch_pick_t<double>(ctx, a, few, bits, cnt, scnt);
+    else launch_pick_t<float>(ctx, a, few, bits, cnt, scnt);
+}
+
 // blocks of a plain trial launch over K hadrons: one per 64 hadrons, at most
 // the resident ones: four hadrons a wave, 16 lanes each, spread over the CUs
 // (1.1 10^4 hadrons: a sampling pass of 245 us; over all CUs 277)
@@ -1806,20 +1839,8 @@ int iss_sample(iss_ctx* ctx, const iss_sample_opts* o, int64_t* n_hadrons) {
     a.slot_species = ctx->d_sp16.p;
     HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
     if (K > 0) {
-        const int pblk = static_cast<int>((Nc + kPickCells - 1) / kPickCells);
-        const bool f64 = ctx->yield_precision == 64;
-        const void* rows = ctx->d_rows.p;
-        uint32_t* gb = learned ? ctx->d_lbits.p : nullptr;
-        uint32_t* gc = learned ? ctx->d_lcnt.p : nullptr;
-        uint32_t* gs = route ? ctx->d_lscnt.p : nullptr;
-        if (f64 && learned)
-            k_pick<double, true><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, true), ctx->stream>>>(a, static_cast<const double*>(rows), row_stride(ctx->Ns, 8), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, ctx->learn_route);
-        else if (f64)
-            k_pick<double, false><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, false), ctx->stream>>>(a, static_cast<const double*>(rows), row_stride(ctx->Ns, 8), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, ctx->learn_route);
-        else if (learned)
-            k_pick<float, true><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, true), ctx->stream>>>(a, static_cast<const float*>(rows), row_stride(ctx->Ns, 4), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, ctx->learn_route);
-        else
-            k_pick<float, false><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, false), ctx->stream>>>(a, static_cast<const float*>(rows), row_stride(ctx->Ns, 4), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, ctx->learn_route);
+        launch_pick(ctx, a, K, learned ? ctx->d_lbits.p : nullptr, learned ? ctx->d_lcnt.p : nullptr,
+                    route ? ctx->d_lscnt.p : nullptr);
         HIPCHK(hipGetLastError());
     }
     int per_cu_trials = 0;
@@ -2536,27 +2557,9 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
             b, cur, D, ctx->d_bevcount.p);
         // every slot's cell and species from its cell's yield row (the FP64
         // prefix in LDS, as one surface's pass); the learned rounds' pairs
-        if (N > 0) {
-            const int pblk = static_cast<int>((N + kPickCells - 1) / kPickCells);
-            const bool f64 = ctx->yield_precision == 64;
-            const void* rows = ctx->d_rows.p;
-            uint32_t* gb = learned ? ctx->d_lbits.p : nullptr;
-            uint32_t* gc = learned ? ctx->d_lcnt.p : nullptr;
-            uint32_t* gs = route ? ctx->d_lscnt.p : nullptr;
-            const int thr = ctx->learn_route;
-            if (f64 && learned)
-                k_pick<double, true><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, true), ctx->stream>>>(
-                    a, static_cast<const double*>(rows), row_stride(ctx->Ns, 8), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, thr);
-            else if (f64)
-                k_pick<double, false><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, false), ctx->stream>>>(
-                    a, static_cast<const double*>(rows), row_stride(ctx->Ns, 8), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, thr);
-            else if (learned)
-                k_pick<float, true><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, true), ctx->stream>>>(
-                    a, static_cast<const float*>(rows), row_stride(ctx->Ns, 4), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, thr);
-            else
-                k_pick<float, false><<<pblk, kWave * kPickCells, pick_lds_bytes(ctx->Ns, false), ctx->stream>>>(
-                    a, static_cast<const float*>(rows), row_stride(ctx->Ns, 4), ctx->d_sp16.p, ctx->d_cellidx.p, gb, gc, gs, thr);
-        }
+        if (N > 0)
+            launch_pick(ctx, a, setup_cap, learned ? ctx->d_lbits.p : nullptr, learned ? ctx->d_lcnt.p : nullptr,
+                        route ? ctx->d_lscnt.p : nullptr);
         if (!learned) {
             k_setup<true><<<setup_blocks, 256, 0, ctx->stream>>>(a, ctx->d_setup.p, nullptr, nullptr);
             k_trials<<<nblk_trials, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);

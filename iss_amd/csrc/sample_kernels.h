@@ -542,6 +542,136 @@ __global__ __launch_bounds__(kWave * kPickCells) void k_pick(SampleArgs a, const
     }
 }
 
+// The same choices where cells hold few slots (a batched round: about 0.5
+// each): a wave takes kPickSpan consecutive cells and skips the empty ones.
+// Lane q draws for slot q of the wave's (64 at a time); a cell's prefix stays
+// in registers, its row is loaded while the cell before it is drawn, and its
+// slots follow one another: the first lane with an entry above the draw.
+// The general kernel starts a wave for every empty cell, draws 64 lanes'
+// Philox blocks for one slot and searches LDS.  What bounds this one is vector
+// issue, about 150 instructions a cell (450 with the lanes' bounds as
+// conditions instead of the buffer's, and G a run-time value).
+constexpr int kPickSpan = 16;
+template <typename R, int G>
+__global__ __launch_bounds__(kWave * kPickCells, 8) void k_pick_few(const int64_t* __restrict__ off, int64_t Nc, int Ns,
+                                                                 uint64_t seed, uint32_t chunk0,
+                                                                 const uint32_t* __restrict__ chunk_dev,
+                                                                 int64_t setup_cap, const R* __restrict__ rows,
+                                                                 int stride, uint16_t* __restrict__ sp16,
+                                                                 uint32_t* __restrict__ cellidx) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int64_t c0 = (static_cast<int64_t>(blockIdx.x) * kPickCells + w) * kPickSpan;
+    if (c0 >= Nc) return;  // whole waves; no workgroup barrier below
+    const uint32_t chunk = chunk_dev ? *chunk_dev : chunk0;
+    const int nc = static_cast<int>(min<int64_t>(kPickSpan, Nc - c0));
+    const int flast = (Ns - 1) / G, klast = (Ns - 1) % G;
+    // lane i: the wave's first slot of cell c0 + i (lane nc: of the next wave;
+    // a pass has less than 2^31 slots)
+    const int64_t off_l = off[c0 + min(lane, nc)];
+    const int64_t beg = readlane64(off_l, 0);
+    // (batched rounds: only the slots with set-up records)
+    const int64_t q_lim = setup_cap > 0 ? max<int64_t>(0, setup_cap - beg) : INT64_MAX;
+    const int q_l = static_cast<int>(min(off_l - beg, q_lim));
+    const int total = __builtin_amdgcn_readlane(q_l, nc);
+    const int q_n = __shfl_down(q_l, 1, kWave);
+    for (int qb = 0; qb < total; qb += kWave) {
+        const int q = qb + lane;
+        int icell = 0;
+        for (int i = 1; i < nc; i++) icell += (q >= __builtin_amdgcn_readlane(q_l, i)) ? 1 : 0;
+        Stream st(seed, static_cast<uint32_t>(c0 + icell), static_cast<uint32_t>(q - __shfl(q_l, icell)),
+                  tag_word(TAG_SETUP, chunk));
+        const double u = st.uniform();
+        int mine = 0;
+        // the cells with slots among these 64
+        unsigned long long todo = __ballot(lane < nc && q_n > q_l && q_n > qb && q_l < qb + kWave);
+        // lane l's species l G .. l G + G - 1 of a row; zero beyond the row
+        // (the buffer's bounds)
+        R yr[G];
+        auto load = [&](int i) {
+            const R* row = rows + (c0 + i) * stride;
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<R*>(row), 0, Ns * static_cast<int>(sizeof(R)),
+                                                                0x00020000);
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const int at = (lane * G + k) * static_cast<int>(sizeof(R));
+                if constexpr (sizeof(R) == 8)
+                    yr[k] = __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0));
+                else
+                    yr[k] = __builtin_bit_cast(R, __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0));
+            }
+        };
+        if (todo) load(__builtin_ctzll(todo));
+        while (todo) {
+            const int i = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            double v[G];
+            double acc = 0.;
+            uint32_t mb = 0u;  // bit k: the lane's species k has a positive yield
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+                const double y = static_cast<double>(yr[k]);
+                acc += y;
+                v[k] = acc;
+                mb |= (y > 0.) ? (1u << k) : 0u;
+            }
+            if (todo) load(__builtin_ctzll(todo));
+            // the running maximum of the earlier lanes' last values is the
+            // lane before's, where every lane's first entry is no less
+            const double base = dpp_f64<kDppWaveShr1>(0., wave_scan_dpp(acc));
+            const double last = base + acc;
+            double lmax = dpp_f64<kDppWaveShr1>(0., last);
+            if (__ballot(lane <= flast && !(lmax <= base + v[0])))
+                lmax = dpp_f64<kDppWaveShr1>(0., wave_max_scan_dpp(last));
+#pragma unroll
+            for (int k = 0; k < G; k++) v[k] = fmax(base + v[k], lmax);
+            const double x_l = u * readlane64(fmax(last, lmax), flast);
+            const unsigned long long some = __ballot(mb != 0u);
+            const int r0 = max(__builtin_amdgcn_readlane(q_l, i) - qb, 0);
+            const int r1 = min(__builtin_amdgcn_readlane(q_n, i) - qb, kWave);
+            for (int r = r0; r < r1; r++) {
+                // the first entry above the draw
+                const double x = readlane64(x_l, r);
+                int m = 0;
+#pragma unroll
+                for (int k = 0; k < G; k++) m += !(x < v[k]) ? 1 : 0;
+                // (a lane's entries past the last species repeat its last one,
+                // and so do not hit; lanes past the last species do not count)
+                const unsigned long long hit = __ballot(m < G) & (~0ull >> (63 - flast));
+                int f = flast, k = klast;
+                if (hit) {
+                    f = __builtin_ctzll(hit);
+                    k = __builtin_amdgcn_readlane(m, f);
+                }
+                const uint32_t bits = __builtin_amdgcn_readlane(static_cast<int>(mb), f);
+                if (!((bits >> k) & 1u)) {
+                    // the nearest species of positive yield, first upwards
+                    const unsigned long long up = f < 63 ? some >> (f + 1) << (f + 1) : 0ull;
+                    const unsigned long long dn = some & ((1ull << f) - 1);
+                    const uint32_t bu = bits >> k << k, bd = bits & ((1u << k) - 1);
+                    if (bu) {
+                        k = __builtin_ctz(bu);
+                    } else if (up) {
+                        f = __builtin_ctzll(up);
+                        k = __builtin_ctz(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mb), f)));
+                    } else if (bd) {
+                        k = 31 - __builtin_clz(bd);
+                    } else if (dn) {
+                        f = 63 - __builtin_clzll(dn);
+                        k = 31 - __builtin_clz(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mb), f)));
+                    } else {
+                        f = k = 0;
+                    }
+                }
+                mine = lane == r ? f * G + k : mine;
+            }
+        }
+        if (q < total) {
+            sp16[beg + q] = static_cast<uint16_t>(mine);
+            cellidx[beg + q] = static_cast<uint32_t>(c0 + icell);
+        }
+    }
+}
+
 // an empty record (out of trials, or outside the momentum tables); batched
 // rounds count a slot beyond the reserved output instead of writing it
 __device__ __forceinline__ void write_hole(const SampleArgs& a, uint64_t outp) {
