@@ -8,11 +8,15 @@
 // n_k(r) = clamp(E_k - r R, 0, R) events.  One round is
 //   k_batch_counts        Poisson(n_k(r) N_c) hadrons per cell
 //   scan                  round-local hadron offsets (all surfaces at once)
-//   k_batch_roots         per surface: its hadron block, its permutation
-//   k_batch_multi_*       per surface: Multinomial over its n_k(r) events
+//   k_batch_roots         per surface: its hadron block, its permutation; the
+//                         round and output base of the kernels after it, and
+//                         those of the next round
 //   k_setup, k_trials     the one-surface kernels, reading the round, the
 //                         hadron count and the output base from the device
-//   k_batch_advance       output base += hadrons of the round, round += 1
+// and after the rounds, for all of them at once (a level of the binomial tree
+// is a chain of 13-20 us whatever its number of nodes: 15 rounds of 48
+// surfaces 850 us in the rounds, 85 after them),
+//   k_batch_multi_*       per (round, surface): Multinomial over its events
 // Every size the kernels need lives on the device, so the host captures one
 // round into a hipGraph and replays it for all rounds (no host round trip,
 // no memset inside the graph).  The output is round-major, then surface, then
@@ -33,8 +37,8 @@ struct BatchDev {
     const int32_t* events;          // [S] events of each surface
     int S;
     int R;                          // events per surface per round
-    uint32_t* round;                // current round (device)
-    unsigned long long* out_base;   // hadrons written by earlier rounds (device)
+    uint32_t* round;                // [2] (device): the round to count, the round being sampled
+    unsigned long long* out_base;   // [2] (device): hadrons counted so far, before the round being sampled
     double ymult;                   // y_RB - y_LB for boost-invariant surfaces, else 1
 };
 
@@ -58,37 +62,48 @@ __global__ void k_batch_counts(BatchDev b, const double* __restrict__ ctot, int6
     counts[c] = static_cast<uint32_t>(min<int64_t>(cnt, 0xFFFFFFFFll));
 }
 
-// per surface: the root of its event tree (its hadrons this round), the keyed
+// per surface: the root of its event tree (its hadrons of the round), the keyed
 // permutation of its block and the output segment of (round, surface)
-__global__ void k_batch_roots(BatchDev b, const int64_t* __restrict__ off, uint64_t seed,
-                              int64_t* __restrict__ tree, Permutation* __restrict__ perms,
-                              int64_t* __restrict__ seg) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= b.S) return;
-    const uint32_t r = *b.round;
-    const int64_t h0 = off[b.surf_off[k]], h1 = off[b.surf_off[k + 1]];
-    const int64_t H = h1 - h0;
-    tree[k] = H;
-    Permutation p;
-    p.init(static_cast<uint64_t>(H > 0 ? H : 1),
-           seed ^ (0x5851F42D4C957F2Dull * (static_cast<uint64_t>(k) + 1)) ^ (static_cast<uint64_t>(r) << 40));
-    perms[k] = p;
-    const int64_t at = 2 * (static_cast<int64_t>(r) * b.S + k);
-    seg[at] = static_cast<int64_t>(*b.out_base) + h0;
-    seg[at + 1] = H;
+__global__ __launch_bounds__(256) void k_batch_roots(BatchDev b, const int64_t* __restrict__ off, int64_t N,
+                                                    uint64_t seed, int64_t* __restrict__ tree,
+                                                    Permutation* __restrict__ perms, int64_t* __restrict__ seg) {
+    // (one workgroup: round and base advance once every thread has read them)
+    const uint32_t r = b.round[0];
+    const unsigned long long out0 = b.out_base[0];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        b.round[0] = r + 1;
+        b.round[1] = r;
+        b.out_base[0] = out0 + static_cast<unsigned long long>(off[N]);
+        b.out_base[1] = out0;
+    }
+    for (int k = threadIdx.x; k < b.S; k += blockDim.x) {
+        const int64_t h0 = off[b.surf_off[k]], h1 = off[b.surf_off[k + 1]];
+        const int64_t H = h1 - h0;
+        const int64_t at = static_cast<int64_t>(r) * b.S + k;
+        tree[at] = H;
+        Permutation p;
+        p.init(static_cast<uint64_t>(H > 0 ? H : 1),
+               seed ^ (0x5851F42D4C957F2Dull * (static_cast<uint64_t>(k) + 1)) ^ (static_cast<uint64_t>(r) << 40));
+        perms[k] = p;
+        seg[2 * at] = static_cast<int64_t>(out0) + h0;
+        seg[2 * at + 1] = H;
+    }
 }
 
-// level d of every surface's binomial tree: node (k, j) covers the events
-// [j n / 2^d, (j + 1) n / 2^d) of surface k's n = n_k(r)
-__global__ void k_batch_multi_level(BatchDev b, const int64_t* __restrict__ parent, int64_t* __restrict__ child,
-                                    int d, uint64_t seed) {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= (static_cast<int64_t>(b.S) << d)) return;
+// level d of every (round, surface)'s binomial tree: node (r, k, j) covers the
+// events [j n / 2^d, (j + 1) n / 2^d) of surface k's n = n_k(r)
+__global__ void k_batch_multi_level(BatchDev b, int rounds, const int64_t* __restrict__ parent,
+                                    int64_t* __restrict__ child, int d, uint64_t seed) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t nodes = static_cast<int64_t>(b.S) << d;  // of a round
+    if (i >= nodes * rounds) return;
+    const uint32_t r = static_cast<uint32_t>(i / nodes);
+    const int64_t t = i - r * nodes;
     const int k = static_cast<int>(t >> d);
     const int64_t j = t & ((1ll << d) - 1);
-    const uint32_t r = *b.round;
     const int64_t E = round_events(b.events[k], r, b.R);
-    const int64_t n = parent[t];
+    const int64_t n = parent[i];
     const int64_t lo = (j * E) >> d, hi = ((j + 1) * E) >> d;
     const int64_t mid = ((2 * j + 1) * E) >> (d + 1);
     int64_t nl = 0;
@@ -97,35 +112,31 @@ __global__ void k_batch_multi_level(BatchDev b, const int64_t* __restrict__ pare
         Stream st(seed, static_cast<uint32_t>(t), static_cast<uint32_t>(d), tag_word(TAG_MULTI, r));
         nl = binomial(n, p, st);
     }
-    child[2 * t] = nl;
-    child[2 * t + 1] = n - nl;
+    child[2 * i] = nl;
+    child[2 * i + 1] = n - nl;
 }
 
 // leaves (2^D >= R): event sizes of (round, surface)
-__global__ void k_batch_multi_leaves(BatchDev b, const int64_t* __restrict__ leaf, int D,
+__global__ void k_batch_multi_leaves(BatchDev b, int rounds, const int64_t* __restrict__ leaf, int D,
                                      uint32_t* __restrict__ evcount) {
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= (static_cast<int64_t>(b.S) << D)) return;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t nodes = static_cast<int64_t>(b.S) << D;
+    if (i >= nodes * rounds) return;
+    const uint32_t r = static_cast<uint32_t>(i / nodes);
+    const int64_t t = i - r * nodes;
     const int k = static_cast<int>(t >> D);
     const int64_t j = t & ((1ll << D) - 1);
-    const uint32_t r = *b.round;
     const int64_t E = round_events(b.events[k], r, b.R);
     const int64_t lo = (j * E) >> D, hi = ((j + 1) * E) >> D;
     if (hi - lo == 1)
-        evcount[(static_cast<int64_t>(r) * b.S + k) * b.R + lo] = static_cast<uint32_t>(leaf[t]);
-}
-
-__global__ void k_batch_advance(BatchDev b, const int64_t* __restrict__ off, int64_t N) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *b.out_base += static_cast<unsigned long long>(off[N]);
-        *b.round += 1u;
-    }
+        evcount[(static_cast<int64_t>(r) * b.S + k) * b.R + lo] = static_cast<uint32_t>(leaf[i]);
 }
 
 // per-surface sums of the per-cell totals (one block per surface, FP64)
-__global__ __launch_bounds__(256) void k_batch_lambda(const int64_t* __restrict__ surf_off,
+constexpr int kLambdaThreads = 1024;
+__global__ __launch_bounds__(kLambdaThreads) void k_batch_lambda(const int64_t* __restrict__ surf_off,
                                                      const double* __restrict__ ctot, double* __restrict__ lam) {
-    __shared__ double ws[256 / kWave];
+    __shared__ double ws[kLambdaThreads / kWave];
     const int k = blockIdx.x;
     double s = 0.;
     for (int64_t c = surf_off[k] + threadIdx.x; c < surf_off[k + 1]; c += blockDim.x) s += ctot[c];
@@ -134,7 +145,7 @@ __global__ __launch_bounds__(256) void k_batch_lambda(const int64_t* __restrict_
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.;
-        for (int w = 0; w < 256 / kWave; w++) t += ws[w];
+        for (int w = 0; w < kLambdaThreads / kWave; w++) t += ws[w];
         lam[k] = t;
     }
 }

@@ -462,12 +462,18 @@ void clear_routed_stats(iss_ctx* ctx) {
     ctx->stats.n_routed_inner = 0;
 }
 
-int launch_scan(iss_ctx* ctx, const uint32_t* in, int64_t n, int64_t* out) {
+// the launches alone (sums: room for the tile sums and their total)
+void enqueue_scan(iss_ctx* ctx, const uint32_t* in, int64_t n, int64_t* sums, int64_t* out) {
     const int64_t ntiles = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
-    HIPCHK(ctx->d_scan.ensure(ntiles + 1));
-    k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(in, n, ctx->d_scan.p);
-    k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(ctx->d_scan.p, ntiles);
-    k_scan_apply<<<ntiles, kScanBlock, 0, ctx->stream>>>(in, n, ctx->d_scan.p, out);
+    const bool direct = ntiles <= kScanDirect;
+    if (ntiles > 1) k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(in, n, sums);
+    if (!direct) k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(sums, ntiles);
+    k_scan_apply<<<ntiles, kScanBlock, 0, ctx->stream>>>(in, n, sums, direct ? 1 : 0, out);
+}
+
+int launch_scan(iss_ctx* ctx, const uint32_t* in, int64_t n, int64_t* out) {
+    HIPCHK(ctx->d_scan.ensure(std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile) + 1));
+    enqueue_scan(ctx, in, n, ctx->d_scan.p, out);
     HIPCHK(hipGetLastError());
     return ISS_OK;
 }
@@ -2424,7 +2430,7 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
         const int rc = ensure_tcell(ctx);
         if (rc) return rc;
     }
-    k_batch_lambda<<<S, 256, 0, ctx->stream>>>(ctx->d_surf_off.p, ctx->d_ctot.p, ctx->d_lam.p);
+    k_batch_lambda<<<S, kLambdaThreads, 0, ctx->stream>>>(ctx->d_surf_off.p, ctx->d_ctot.p, ctx->d_lam.p);
     HIPCHK(hipGetLastError());
     std::vector<double> lam(S);
     HIPCHK(hipMemcpyAsync(lam.data(), ctx->d_lam.p, sizeof(double) * S, hipMemcpyDeviceToHost, ctx->stream));
@@ -2454,13 +2460,13 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     HIPCHK(ctx->d_perms.ensure(S));
     HIPCHK(ctx->d_seg.ensure(2 * static_cast<size_t>(std::max(rounds, 1)) * S));
     HIPCHK(ctx->d_bevcount.ensure(static_cast<size_t>(std::max(rounds, 1)) * S * R));
-    HIPCHK(ctx->d_tree0.ensure(static_cast<size_t>(S) << D));
-    HIPCHK(ctx->d_tree1.ensure(static_cast<size_t>(S) << D));
+    HIPCHK(ctx->d_tree0.ensure((static_cast<size_t>(S) << D) * std::max(rounds, 1)));
+    HIPCHK(ctx->d_tree1.ensure((static_cast<size_t>(S) << D) * std::max(rounds, 1)));
     HIPCHK(ctx->d_scan.ensure(std::max<int64_t>(1, (N + kScanTile - 1) / kScanTile) + 1));
-    HIPCHK(ctx->d_bround.ensure(1));
-    HIPCHK(ctx->d_bbase.ensure(1));
-    HIPCHK(hipMemsetAsync(ctx->d_bround.p, 0, sizeof(uint32_t), ctx->stream));
-    HIPCHK(hipMemsetAsync(ctx->d_bbase.p, 0, sizeof(unsigned long long), ctx->stream));
+    HIPCHK(ctx->d_bround.ensure(2));
+    HIPCHK(ctx->d_bbase.ensure(2));
+    HIPCHK(hipMemsetAsync(ctx->d_bround.p, 0, 2 * sizeof(uint32_t), ctx->stream));
+    HIPCHK(hipMemsetAsync(ctx->d_bbase.p, 0, 2 * sizeof(unsigned long long), ctx->stream));
     HIPCHK(hipMemsetAsync(ctx->d_stats.p, 0, kStatSlots * sizeof(unsigned long long), ctx->stream));
     BatchDev b{ctx->d_surf_off.p, ctx->d_bevents.p, S, R, ctx->d_bround.p, ctx->d_bbase.p, ymult};
     SampleArgs a = base_args(ctx);
@@ -2471,11 +2477,11 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     a.Kdev = reinterpret_cast<const unsigned long long*>(ctx->d_off.p + N);
     a.seed = o->seed;
     a.chunk = 0;
-    a.chunk_dev = ctx->d_bround.p;
+    a.chunk_dev = ctx->d_bround.p + 1;
     a.surf_off = ctx->d_surf_off.p;
     a.S = S;
     a.perms = ctx->d_perms.p;
-    a.out_base = ctx->d_bbase.p;
+    a.out_base = ctx->d_bbase.p + 1;
     a.out_cap = static_cast<uint64_t>(out_cap);
     a.setup_cap = setup_cap;
     HIPCHK(ctx->d_cellidx.ensure(std::max<int64_t>(setup_cap, 1)));
@@ -2498,7 +2504,6 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     if (ctx->blocks_per_cu[0] > 0) per_cu = std::min(ctx->blocks_per_cu[0], per_cu);
     const int nblk_trials = ctx->num_cu * per_cu;
     const int setup_blocks = ctx->num_cu * 8;
-    const int64_t ntiles = std::max<int64_t>(1, (N + kScanTile - 1) / kScanTile);
     // learned proposal: the round's (cell, species) pairs, one network
     // evaluation and band envelope per pair, the learned trials, and the
     // plain sampler for the hadrons without an envelope; all bounded by the
@@ -2541,20 +2546,9 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     // one round: only kernel launches, every size read on the device
     auto round = [&]() {
         if (N > 0) k_batch_counts<<<(N + 255) / 256, 256, 0, ctx->stream>>>(b, ctx->d_ctot.p, N, o->seed, ctx->d_counts.p);
-        k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_counts.p, N, ctx->d_scan.p);
-        k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(ctx->d_scan.p, ntiles);
-        k_scan_apply<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_counts.p, N, ctx->d_scan.p, ctx->d_off.p);
-        k_batch_roots<<<(S + 63) / 64, 64, 0, ctx->stream>>>(b, ctx->d_off.p, o->seed, ctx->d_tree0.p, ctx->d_perms.p,
-                                                             ctx->d_seg.p);
-        int64_t* cur = ctx->d_tree0.p;
-        int64_t* nxt = ctx->d_tree1.p;
-        for (int d = 0; d < D; d++) {
-            const int64_t nodes = static_cast<int64_t>(S) << d;
-            k_batch_multi_level<<<(nodes + 255) / 256, 256, 0, ctx->stream>>>(b, cur, nxt, d, o->seed);
-            std::swap(cur, nxt);
-        }
-        k_batch_multi_leaves<<<((static_cast<int64_t>(S) << D) + 255) / 256, 256, 0, ctx->stream>>>(
-            b, cur, D, ctx->d_bevcount.p);
+        enqueue_scan(ctx, ctx->d_counts.p, N, ctx->d_scan.p, ctx->d_off.p);
+        k_batch_roots<<<1, 256, 0, ctx->stream>>>(b, ctx->d_off.p, N, o->seed, ctx->d_tree0.p, ctx->d_perms.p,
+                                                  ctx->d_seg.p);
         // every slot's cell and species from its cell's yield row (the FP64
         // prefix in LDS, as one surface's pass); the learned rounds' pairs
         if (N > 0)
@@ -2564,14 +2558,10 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
             k_setup<true><<<setup_blocks, 256, 0, ctx->stream>>>(a, ctx->d_setup.p, nullptr, nullptr);
             k_trials<<<nblk_trials, kTrialThreads, 0, ctx->stream>>>(a, ctx->d_setup.p);
         } else {
-            k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_lcnt.p, N, ctx->d_scan.p);
-            k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(ctx->d_scan.p, ntiles);
-            k_scan_apply<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_lcnt.p, N, ctx->d_scan.p, ctx->d_pairoff.p);
+            enqueue_scan(ctx, ctx->d_lcnt.p, N, ctx->d_scan.p, ctx->d_pairoff.p);
             // routing: the slots of single-hadron pairs head the plain list
             if (route) {
-                k_scan_tiles<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_lscnt.p, N, ctx->d_scan.p);
-                k_scan_top<<<1, kScanBlock, 0, ctx->stream>>>(ctx->d_scan.p, ntiles);
-                k_scan_apply<<<ntiles, kScanBlock, 0, ctx->stream>>>(ctx->d_lscnt.p, N, ctx->d_scan.p, ctx->d_soff.p);
+                enqueue_scan(ctx, ctx->d_lscnt.p, N, ctx->d_scan.p, ctx->d_soff.p);
             }
             const int64_t* soff = route ? ctx->d_soff.p : nullptr;
             const int fblk = static_cast<int>(std::max<int64_t>(1, (N + kPairCellsPerBlock - 1) / kPairCellsPerBlock));
@@ -2587,7 +2577,6 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
                                                                  ctx->d_fb_count.p);
             k_trials_routed<<<ctx->num_cu * (route ? per_cu : per_cu_fb), kTrialThreads, 0, ctx->stream>>>(af, ctx->d_setup.p);
         }
-        k_batch_advance<<<1, 64, 0, ctx->stream>>>(b, ctx->d_off.p, N);
     };
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     if (rounds > 0) {
@@ -2617,6 +2606,19 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
             for (int r = 0; r < rounds; r++) round();
             HIPCHK(hipGetLastError());
         }
+    }
+    if (rounds > 0) {
+        // the event sizes of every (round, surface)
+        int64_t* cur = ctx->d_tree0.p;
+        int64_t* nxt = ctx->d_tree1.p;
+        for (int d = 0; d < D; d++) {
+            const int64_t nodes = (static_cast<int64_t>(S) << d) * rounds;
+            k_batch_multi_level<<<(nodes + 255) / 256, 256, 0, ctx->stream>>>(b, rounds, cur, nxt, d, o->seed);
+            std::swap(cur, nxt);
+        }
+        k_batch_multi_leaves<<<((static_cast<int64_t>(S) << D) * rounds + 255) / 256, 256, 0, ctx->stream>>>(
+            b, rounds, cur, D, ctx->d_bevcount.p);
+        HIPCHK(hipGetLastError());
     }
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
     unsigned long long st[9];

@@ -27,8 +27,13 @@ __global__ void k_counts(const double* __restrict__ ctot, int64_t Nc, double mul
     counts[c] = static_cast<uint32_t>(min<int64_t>(k, 0xFFFFFFFFll));
 }
 
-// ----- exclusive scan of uint32 -> int64 (out[n] = total), 3 phases
+// ----- exclusive scan of uint32 -> int64 (out[n] = total): tile sums, their
+// scan, then the tiles.  One tile is scanned by itself, and up to
+// kScanDirect tiles add the sums before them themselves: a scan of a few
+// thousand entries is one launch, of a million two (each costs 3-5 us on the
+// device and as much on the host).
 constexpr int kScanBlock = 256, kScanItems = 8, kScanTile = kScanBlock * kScanItems;
+constexpr int64_t kScanDirect = 1024;
 
 __device__ __forceinline__ int64_t block_exclusive_scan(int64_t v, int64_t* total) {
     __shared__ int64_t wsum[kScanBlock / kWave];
@@ -75,8 +80,9 @@ __global__ void k_scan_top(int64_t* __restrict__ tile_sums, int64_t ntiles) {
     if (threadIdx.x == 0) tile_sums[ntiles] = carry_s;
 }
 
+// tile_sums: the scanned tile sums, with `direct` the sums themselves
 __global__ void k_scan_apply(const uint32_t* __restrict__ in, int64_t n,
-                             const int64_t* __restrict__ tile_sums, int64_t* __restrict__ out) {
+                             const int64_t* __restrict__ tile_sums, int direct, int64_t* __restrict__ out) {
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile + threadIdx.x * kScanItems;
     int64_t loc[kScanItems];
     int64_t v = 0;
@@ -84,13 +90,20 @@ __global__ void k_scan_apply(const uint32_t* __restrict__ in, int64_t n,
         loc[k] = (base + k < n) ? in[base + k] : 0;
         v += loc[k];
     }
-    int64_t tot;
-    int64_t ex = block_exclusive_scan(v, &tot) + tile_sums[blockIdx.x];
+    int64_t before = 0, tot;
+    if (direct) {
+        int64_t p = 0;
+        for (unsigned i = threadIdx.x; i < blockIdx.x; i += kScanBlock) p += tile_sums[i];
+        block_exclusive_scan(p, &before);
+    } else {
+        before = tile_sums[blockIdx.x];
+    }
+    int64_t ex = block_exclusive_scan(v, &tot) + before;
     for (int k = 0; k < kScanItems; k++) {
         if (base + k < n) out[base + k] = ex;
         ex += loc[k];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = tile_sums[gridDim.x];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
 }
 
 // ----- hadrons per event: Multinomial(K, 1/E) as a binomial tree.  Level d
