@@ -4,12 +4,12 @@
 // (one translation unit: included by iss_hip.hip)
 //
 // Data-parallel over particles, one generation per pass:
-//   k_decay_pick   per particle: table entry, channel (cumulative branching
-//                  ratio), number of daughters; kind = final (stable or not in
-//                  the table), decayed (2- or 3-body) or gone (other channels:
-//                  no daughters, as in the reference)
+//   k_decay_pick   per sampled hadron: table entry, channel (cumulative
+//                  branching ratio), number of daughters; kind = final (stable
+//                  or not in the table), decayed (2- or 3-body) or gone (other
+//                  channels: no daughters, as in the reference)
 //   scan           daughter offsets of the next generation
-//   k_decay_emit   the daughters, with their parent's index
+//   k_decay_emit   the daughters, with their own choices
 // After the last generation the final particles are placed deterministically
 // without sorting: every particle's count of final descendants is gathered
 // bottom-up from its (contiguous) daughters, a scan over the sampled hadrons
@@ -60,15 +60,18 @@ __device__ __forceinline__ Stream decay_stream(uint64_t seed, int gen, int64_t i
     return Stream(seed, static_cast<uint32_t>(i), static_cast<uint32_t>(i >> 32), tag_word(TAG_DECAY, gen));
 }
 
-// kind, channel and daughter count of every particle of generation `gen`
-// (a channel closed at the pole mass drops the mother and is counted in
-// *nbelow: the reference exits there, src/particle_decay.cpp:351-357, 431-441)
-__global__ void k_decay_pick(DecayDev t, const Hadron* __restrict__ P, int64_t n, int gen, uint64_t seed,
-                             uint8_t* __restrict__ kind, int32_t* __restrict__ chan,
-                             uint32_t* __restrict__ nchild, unsigned long long* __restrict__ nbelow) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int e = decay_entry(t, P[i].pid);
+// kind, channel and daughter count of particle i of generation `gen`, of
+// table entry e (a channel closed at the pole mass drops the mother and is
+// counted in *nbelow: the reference exits there, src/particle_decay.cpp:351-357,
+// 431-441)
+struct DecayChoice {
+    uint8_t* __restrict__ kind;
+    int32_t* __restrict__ chan;
+    uint32_t* __restrict__ nchild;
+    unsigned long long* __restrict__ nbelow;
+};
+__device__ __forceinline__ void decay_choose(const DecayDev& t, int e, float mass, int gen, int64_t i, uint64_t seed,
+                                             const DecayChoice& o) {
     uint8_t k = DK_FINAL;
     int c = -1;
     uint32_t nc = 0;
@@ -86,9 +89,9 @@ __global__ void k_decay_pick(DecayDev t, const Hadron* __restrict__ P, int64_t n
                 const int de = t.didx[5 * c + j];
                 msum += static_cast<float>(de >= 0 ? t.mass[de] : 0.);
             }
-            if (static_cast<double>(P[i].mass) < static_cast<double>(msum)) {
+            if (static_cast<double>(mass) < static_cast<double>(msum)) {
                 k = DK_GONE;
-                atomicAdd(nbelow, 1ull);
+                atomicAdd(o.nbelow, 1ull);
             } else {
                 k = DK_DECAYED;
                 nc = static_cast<uint32_t>(np);
@@ -97,9 +100,17 @@ __global__ void k_decay_pick(DecayDev t, const Hadron* __restrict__ P, int64_t n
             k = DK_GONE;
         }
     }
-    kind[i] = k;
-    chan[i] = c;
-    nchild[i] = nc;
+    o.kind[i] = k;
+    o.chan[i] = c;
+    o.nchild[i] = nc;
+}
+
+// the choices of the sampled hadrons; the daughters' are made as they are
+// emitted, where their table entry is at hand (a search of the table, a
+// launch and a pass over the generation less)
+__global__ void k_decay_pick(DecayDev t, const Hadron* __restrict__ P, int64_t n, uint64_t seed, DecayChoice o) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) decay_choose(t, decay_entry(t, P[i].pid), P[i].mass, 0, i, seed, o);
 }
 
 __device__ __forceinline__ void decay_boost(double vx, double vy, double vz, double E, double px, double py,
@@ -115,32 +126,30 @@ __device__ __forceinline__ void decay_boost(double vx, double vy, double vz, dou
     h.pz = static_cast<float>(pz + k * vz);
 }
 
-// daughters of the decayed particles of generation `gen` into generation gen + 1
-__global__ void k_decay_emit(DecayDev t, const Hadron* __restrict__ P, int64_t n, int gen, uint64_t seed,
-                             const uint8_t* __restrict__ kind, const int32_t* __restrict__ chan,
-                             const int64_t* __restrict__ off, Hadron* __restrict__ C, int64_t* __restrict__ parent,
-                             unsigned long long* __restrict__ nfail) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n || kind[i] != DK_DECAYED) return;
+// the NP daughters of particle i of generation `gen`
+template <int NP>
+__device__ __forceinline__ void decay_emit(const DecayDev& t, const Hadron* __restrict__ P, int64_t i, int gen,
+                                           uint64_t seed, int c, int64_t o, Hadron* __restrict__ C,
+                                           const DecayChoice& next, unsigned long long* __restrict__ nfail) {
     const Hadron m = P[i];
-    const int c = chan[i];
     const int e = decay_entry(t, m.pid);
-    const int np = t.npart[c];
     Stream st = decay_stream(seed, gen, i);
     (void)st.uniform();  // the channel draw
-    Hadron d[3];
-    double ms[3];
-    for (int k = 0; k < np; k++) {
+    Hadron d[NP];
+    double ms[NP];
+    int de[NP];
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
         d[k].pid = t.dpid[5 * c + k];
-        const int de = t.didx[5 * c + k];
-        d[k].mass = static_cast<float>(de >= 0 ? t.mass[de] : 0.);
+        de[k] = t.didx[5 * c + k];
+        d[k].mass = static_cast<float>(de[k] >= 0 ? t.mass[de[k]] : 0.);
         ms[k] = d[k].mass;
     }
     const double Mp = m.mass, W = t.width[e];
     const double vx = static_cast<double>(m.px) / m.E, vy = static_cast<double>(m.py) / m.E,
                  vz = static_cast<double>(m.pz) / m.E;
     double life = 1e10;
-    if (np == 2) {
+    if constexpr (NP == 2) {
         const double tt = Mp * Mp - ms[0] * ms[0] - ms[1] * ms[1];
         const double p = sqrt(fmax(tt * tt - 4 * ms[0] * ms[0] * ms[1] * ms[1], 0.)) / (2 * Mp);
         const double phi = st.uniform() * 2 * kPi;
@@ -184,18 +193,63 @@ __global__ void k_decay_emit(DecayDev t, const Hadron* __restrict__ P, int64_t n
         const double q[3][3] = {{-p1 * sth * ck, p1 * sth * sk, p1 * cth},
                                 {t2x * a - t2z * sth * ck, t2x * b + t2z * sth * sk, t2x * cp * sth + t2z * cth},
                                 {t3x * a - t3z * sth * ck, t3x * b + t3z * sth * sk, t3x * cp * sth + t3z * cth}};
+#pragma unroll
         for (int k = 0; k < 3; k++)
             decay_boost(vx, vy, vz, sqrt(ms[k] * ms[k] + q[k][0] * q[k][0] + q[k][1] * q[k][1] + q[k][2] * q[k][2]),
                         q[k][0], q[k][1], q[k][2], d[k]);
     }
-    const int64_t o = off[i];
-    for (int k = 0; k < np; k++) {
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
         d[k].t = static_cast<float>(m.t + life);
         d[k].x = static_cast<float>(m.x + static_cast<double>(m.px) / m.E * life);
         d[k].y = static_cast<float>(m.y + static_cast<double>(m.py) / m.E * life);
         d[k].z = static_cast<float>(m.z + static_cast<double>(m.pz) / m.E * life);
         C[o + k] = d[k];
-        parent[o + k] = i;
+        decay_choose(t, de[k], d[k].mass, gen + 1, o + k, seed, next);
+    }
+}
+
+// Daughters of the decayed particles of generation `gen` into generation
+// gen + 1.  A workgroup lists the two- and three-body decays among its
+// kEmitTile particles in LDS; the first threads take the former, the last
+// threads the latter.  FP64 issue bounds it (some 800 instructions a two-body
+// decay, 2500 a three-body one, sincos, log and divisions), so a thread per
+// particle, whose waves run both for their few decayed lanes, was the slower
+// form: three generations from 4 10^5 hadrons 140 -> 80 us (87 with the
+// daughters' choices, which took 25 in launches of their own).
+constexpr int kEmitThreads = 256, kEmitTile = 512;
+__global__ __launch_bounds__(kEmitThreads, 4) void k_decay_emit(DecayDev t, const Hadron* __restrict__ P, int64_t n,
+                                                            int gen, uint64_t seed,
+                                                            const uint32_t* __restrict__ nchild,
+                                                            const int32_t* __restrict__ chan,
+                                                            const int64_t* __restrict__ off, Hadron* __restrict__ C,
+                                                            DecayChoice next,
+                                                            unsigned long long* __restrict__ nfail) {
+    __shared__ uint16_t list[2][kEmitTile];
+    __shared__ int count[2];
+    if (threadIdx.x < 2) count[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kEmitTile;
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int j = threadIdx.x; j < kEmitTile; j += kEmitThreads) {
+        const uint32_t nc = first + j < n ? nchild[first + j] : 0u;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const unsigned long long m = __ballot(nc == static_cast<uint32_t>(b + 2));
+            int at = 0;
+            if (lane == 0 && m) at = atomicAdd(&count[b], __popcll(m));
+            at = __builtin_amdgcn_readfirstlane(at);
+            if ((m >> lane) & 1ull) list[b][at + __popcll(m & ((1ull << lane) - 1))] = static_cast<uint16_t>(j);
+        }
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < count[0]; q += kEmitThreads) {
+        const int64_t i = first + list[0][q];
+        decay_emit<2>(t, P, i, gen, seed, chan[i], off[i], C, next, nfail);
+    }
+    for (int q = kEmitThreads - 1 - threadIdx.x; q < count[1]; q += kEmitThreads) {
+        const int64_t i = first + list[1][q];
+        decay_emit<3>(t, P, i, gen, seed, chan[i], off[i], C, next, nfail);
     }
 }
 

@@ -265,10 +265,10 @@ struct DecayGen {
     DBuf<uint8_t> kind;
     DBuf<int32_t> chan;
     DBuf<uint32_t> nchild, size;
-    DBuf<int64_t> off, pos, parent;
+    DBuf<int64_t> off, pos;
     void release() {
         own.release(); kind.release(); chan.release(); nchild.release(); size.release();
-        off.release(); pos.release(); parent.release();
+        off.release(); pos.release();
     }
 };
 
@@ -2903,18 +2903,24 @@ int iss_decay(iss_ctx* ctx, uint64_t seed, int64_t* n_hadrons) {
     HIPCHK(ctx->d_stats.ensure(8));
     HIPCHK(hipMemsetAsync(ctx->d_stats.p + 6, 0, 2 * sizeof(unsigned long long), ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    auto choices = [&](DecayGen& G) -> int {
+        HIPCHK(G.kind.ensure(G.n));
+        HIPCHK(G.chan.ensure(G.n));
+        HIPCHK(G.nchild.ensure(G.n));
+        return ISS_OK;
+    };
+    auto choice = [&](DecayGen& G) { return DecayChoice{G.kind.p, G.chan.p, G.nchild.p, ctx->d_stats.p + 6}; };
     for (int g = 0;; g++) {
         DecayGen& G = *gens[g];
         const int64_t n = G.n;
-        HIPCHK(G.kind.ensure(n));
-        HIPCHK(G.chan.ensure(n));
-        HIPCHK(G.nchild.ensure(n));
         HIPCHK(G.size.ensure(n));
         HIPCHK(G.off.ensure(n + 1));
         HIPCHK(G.pos.ensure(n + 1));
-        if (n > 0)
-            k_decay_pick<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->dec, G.P, n, g, seed, G.kind.p, G.chan.p,
-                                                                   G.nchild.p, ctx->d_stats.p + 6);
+        if (g == 0) {
+            if (int rc = choices(G)) return rc;
+            if (n > 0)
+                k_decay_pick<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->dec, G.P, n, seed, choice(G));
+        }
         HIPCHK(hipGetLastError());
         int rc = launch_scan(ctx, G.nchild.p, n, G.off.p);
         if (rc) return rc;
@@ -2928,11 +2934,12 @@ int iss_decay(iss_ctx* ctx, uint64_t seed, int64_t* n_hadrons) {
         ngen = g + 2;
         DecayGen& H = *gens[g + 1];
         HIPCHK(H.own.ensure(nn));
-        HIPCHK(H.parent.ensure(nn));
         H.P = H.own.p;
         H.n = nn;
-        k_decay_emit<<<(n + 255) / 256, 256, 0, ctx->stream>>>(ctx->dec, G.P, n, g, seed, G.kind.p, G.chan.p,
-                                                               G.off.p, H.own.p, H.parent.p, ctx->d_stats.p + 7);
+        if ((rc = choices(H))) return rc;
+        k_decay_emit<<<(n + kEmitTile - 1) / kEmitTile, kEmitThreads, 0, ctx->stream>>>(
+            ctx->dec, G.P, n, g, seed, G.nchild.p, G.chan.p, G.off.p, H.own.p, choice(H),
+            ctx->d_stats.p + 7);
         HIPCHK(hipGetLastError());
     }
     // final descendants, bottom-up
