@@ -3,15 +3,18 @@
 // Pipeline per context (all on one HIP stream):
 //   k_lab_to_lrf + k_compact  regulation and rest-frame transform of the surface
 //   k_cell_prep               per-cell delta-f coefficients (FP64)
-//   k_yield<R, MODE>          per-(cell, species) yields, the FP64 species CDF of
-//                             every cell and per-block FP64 species partials
+//   k_yield_rows<R, ...>      per-(cell, species) yields as rows, cell totals and
+//                             species partials (k_yield: the FP64 CDF layout)
 //   k_species_reduce          FP64 per-species totals
 //   k_counts                  hadrons per cell over all events: Poisson(E * N_c)
 //   scan                      cell offsets (int64)
-//   k_multinomial_level       hadrons per event: Multinomial(K, 1/E), binomial tree
-//   k_sample                  species pick, LRF momentum rejection, boost, output
-//   k_spectra_rec + k_spectra smooth dN/(pT dpT dphi dy) on a (pT, phi) grid
-//                             (+ k_spectra_reduce), host-side flows
+//   k_event_hist              hadrons per event (many events: a binomial tree)
+//   k_pick, k_pick_few        species and cell of every hadron slot
+//   k_setup                   |p| table, normalisation and output slot
+//   k_trials                  LRF momentum rejection, boost, output
+//   k_spectra_rec + k_spectra64 / k_spectra32 (integrated over eta_s),
+//   k_spectra_y / k_spectra_points (per rapidity): smooth dN/(pT dpT dphi dy) on
+//                             a (pT, phi) grid (+ k_spectra_reduce), host-side flows
 //
 // Poisson splitting: the reference draws N_{e,s} ~ Poisson(sum_c N_{c,s}) per
 // event and species and then a cell per hadron from the species' cell CDF

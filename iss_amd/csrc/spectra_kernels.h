@@ -498,7 +498,7 @@ __global__ __launch_bounds__(64) void k_spectra_y(SpectraArgs a) {
 // The FP64 spectra of mode 0 are VALU-bound: N cells x n_eta nodes x points
 // evaluations of one integrand, so its FP64 instruction count is the time.
 // The kernel below evaluates the same sums with about 40 FP64 issue slots a
-// point where the rest-frame form (k_spectra) takes about 110:
+// point where the rest-frame form takes about 110:
 //   * Everything the integrand contracts is linear or quadratic in the lab
 //     momentum (mT cosh y, px, py, mT sinh y), and cosh, sinh of
 //     y = eta_cell + (y - eta_s)_k are linear in those of the node.  So per
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(64) void k_spectra_y(SpectraArgs a) {
 //     with its rounding) and an exponent shift, the reciprocal of the
 //     occupancy a hardware estimate with one third-order step (1 ulp).
 // Measured at 200,000 cells x 3 species x 720 points x 81 nodes: 98.8 ms
-// with k_spectra<double>, 40.5 ms with this kernel (8.6e11 points/s,
+// with the rest-frame form, 40.5 ms with this kernel (8.6e11 points/s,
 // 31 of the 39 TFMA/s of the FP64 vector unit).
 constexpr int kMilneRec = 48;
 enum MilneSlot {
