@@ -131,8 +131,8 @@ struct DBuf {
 // Pinned host memory for the read-backs of counts, flags and totals: a copy
 // from device memory into pageable memory goes through the runtime's staging
 // buffer and costs tens of microseconds more than one into pinned memory.
-// Slots: PIN_OOB int, PIN_K int64, PIN_STATS 16 x u64, PIN_AUX 2 x int64, then
-// PIN_MU int, PIN_TOT [Ns] doubles.
+// Slots: PIN_K int64, PIN_STATS 16 x u64, PIN_AUX 2 x int64, then
+// PIN_MU int, PIN_TOT [Ns] doubles and an int (the out-of-table flag).
 struct PinBuf {
     void* p = nullptr;
     size_t cap = 0;
@@ -154,7 +154,7 @@ struct PinBuf {
     template <typename T>
     T* at(size_t off) { return reinterpret_cast<T*>(static_cast<char*>(p) + off); }
 };
-constexpr size_t PIN_OOB = 0, PIN_K = 8, PIN_STATS = 64, PIN_AUX = 192, PIN_MU = 208, PIN_TOT = 256;
+constexpr size_t PIN_K = 8, PIN_STATS = 64, PIN_AUX = 192, PIN_MU = 208, PIN_TOT = 256;
 // device counters: [0..3] trials, |p| proposals, failed, out of table; [4..5]
 // learned fallback and envelope violations; [6..7] batch overflow flags; [8]
 // routed hadrons of batches; [9..12] the routed plain trials' [0..3]
@@ -350,7 +350,6 @@ struct iss_ctx {
     bool charges_outside = false;  // a species charge beyond the row pass's fugacity rows
     DBuf<RowSpD> d_rowspd;     // the same in FP64, [2][row_stride(Ns, 8)]
     DBuf<double> d_cdf, d_ctot, d_ctot_part, d_partial, d_stot;
-    DBuf<int> d_oob;
     DBuf<char> d_raw;
     // sampling
     DBuf<uint32_t> d_counts, d_evcount;
@@ -823,7 +822,7 @@ int run_yields(iss_ctx* ctx, int precision, void* per_cell_host, double* totals_
     if (rowsl) HIPCHK(ctx->d_rows.ensure(std::max<int64_t>(1, Nc) * stride * esz));
     else HIPCHK(ctx->d_cdf.ensure(std::max<int64_t>(1, Nc) * cdf_stride(Ns)));
     HIPCHK(ctx->d_ctot.ensure(std::max<int64_t>(1, Nc)));
-    HIPCHK(ctx->d_stot.ensure(Ns));
+    HIPCHK(ctx->d_stot.ensure(Ns + 1));  // the species totals, then the out-of-table flag: one read-back
     // partials sized for the largest grid the launches use
     const int max_blk = ctx->num_cu * kPartialBlocksPerCU;
     HIPCHK(ctx->d_partial.ensure(static_cast<size_t>(max_blk) * Ns));
@@ -837,9 +836,8 @@ int run_yields(iss_ctx* ctx, int precision, void* per_cell_host, double* totals_
     a.partial = ctx->d_partial.p;
     a.ycol = ycol;
     a.rows = rowsl ? static_cast<void*>(ctx->d_rows.p) : nullptr;
-    HIPCHK(ctx->d_oob.ensure(1));
-    a.oob = ctx->d_oob.p;
-    HIPCHK(hipMemsetAsync(ctx->d_oob.p, 0, sizeof(int), ctx->stream));
+    a.oob = reinterpret_cast<int*>(ctx->d_stot.p + Ns);
+    HIPCHK(hipMemsetAsync(a.oob, 0, sizeof(int), ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     int nblk = 1;
     if (Nc > 0 && ctx->df.include_diffusion) {
@@ -851,9 +849,9 @@ int run_yields(iss_ctx* ctx, int precision, void* per_cell_host, double* totals_
     // the pass, the species reduction and the read-backs, then one wait; a
     // Bessel argument outside the table (flag oob) reruns the pass with the
     // exact fallback
-    HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * Ns));
-    int* h_oob = ctx->h_pin.at<int>(PIN_OOB);
+    HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * (Ns + 1)));
     double* h_tot = ctx->h_pin.at<double>(PIN_TOT);
+    const int* h_oob = reinterpret_cast<const int*>(h_tot + Ns);
     for (int exact = 0; exact < 2; exact++) {
         if (Nc > 0) {
             int rc;
@@ -879,9 +877,11 @@ int run_yields(iss_ctx* ctx, int precision, void* per_cell_host, double* totals_
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
         const bool check = Nc > 0 && !exact;
-        if (check) HIPCHK(hipMemcpyAsync(h_oob, ctx->d_oob.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         if (totals_host)
-            HIPCHK(hipMemcpyAsync(h_tot, ctx->d_stot.p, sizeof(double) * Ns, hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(hipMemcpyAsync(h_tot, ctx->d_stot.p, sizeof(double) * Ns + sizeof(int), hipMemcpyDeviceToHost,
+                                  ctx->stream));
+        else if (check)
+            HIPCHK(hipMemcpyAsync(h_tot + Ns, a.oob, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         if (per_cell_host && Nc > 0) {
             if (rowsl)  // the rows without their padding
                 HIPCHK(hipMemcpy2DAsync(per_cell_host, esz * Ns, ctx->d_rows.p, esz * stride, esz * Ns, Nc,
@@ -1199,7 +1199,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_ktab.release(); ctx->d_ktabf.release(); ctx->d_ptab.release();
     ctx->d_cells.release(); ctx->d_tmp.release(); ctx->d_lab.release(); ctx->d_coef.release(); ctx->d_u32.release();
     ctx->d_i64.release(); ctx->d_mu_used.release(); ctx->d_scan.release(); ctx->d_eos.release(); ctx->d_cdf.release();
-    ctx->d_ctot.release(); ctx->d_ctot_part.release(); ctx->d_rowspd.release(); ctx->d_partial.release(); ctx->d_oob.release(); ctx->d_stot.release(); ctx->d_raw.release();
+    ctx->d_ctot.release(); ctx->d_ctot_part.release(); ctx->d_rowspd.release(); ctx->d_partial.release(); ctx->d_stot.release(); ctx->d_raw.release();
     ctx->d_counts.release(); ctx->d_evcount.release(); ctx->d_off.release(); ctx->d_evoff.release();
     ctx->d_tree0.release(); ctx->d_tree1.release(); ctx->d_out.release(); ctx->d_setup.release(); ctx->d_stats.release();
     ctx->d_cellidx.release(); ctx->d_tcell.release(); ctx->d_tspec.release();
