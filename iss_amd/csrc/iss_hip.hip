@@ -34,6 +34,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <string>
 #include <thread>
 #include <tuple>
@@ -1059,16 +1060,24 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     // the 321 UrQMD species where mu_S = mu_Q = 0; 314 with all potentials).
     // A charge matters where its potential is not zero on every cell, or
     // where it multiplies a bulk or diffusion term.
-    HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * ctx->Ns));
-    HIPCHK(ctx->d_mu_used.ensure(1));
-    HIPCHK(hipMemsetAsync(ctx->d_mu_used.p, 0, sizeof(int), ctx->stream));
-    k_mu_used<<<static_cast<int>(std::min<int64_t>((N + 1023) / 1024, 256)), 256, 0, ctx->stream>>>(rec, N,
-                                                                                                     ctx->d_mu_used.p);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(ctx->h_pin.at<int>(PIN_MU), ctx->d_mu_used.p, sizeof(int), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    const int mu_used = *ctx->h_pin.at<int>(PIN_MU);
+    // Without two species of one mass and statistics (one species, or a few
+    // identified ones) none can share, and the surface is not asked: 15 us of a
+    // small call.
+    std::set<std::pair<double, int>> masses;
+    for (int i = 0; i < ns; i++) masses.emplace(ctx->h_sp[species[i]].mass, ctx->h_sp[species[i]].sign);
+    int mu_used = 0;
+    if (static_cast<int64_t>(masses.size()) < ns) {
+        HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * ctx->Ns));
+        HIPCHK(ctx->d_mu_used.ensure(1));
+        HIPCHK(hipMemsetAsync(ctx->d_mu_used.p, 0, sizeof(int), ctx->stream));
+        k_mu_used<<<static_cast<int>(std::min<int64_t>((N + 1023) / 1024, 256)), 256, 0, ctx->stream>>>(rec, N,
+                                                                                                         ctx->d_mu_used.p);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(ctx->h_pin.at<int>(PIN_MU), ctx->d_mu_used.p, sizeof(int), hipMemcpyDeviceToHost,
+                              ctx->stream));
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+        mu_used = *ctx->h_pin.at<int>(PIN_MU);
+    }
     const bool c22 = bulk == BULK_22MOM;
     const bool by_B = (mu_used & MU_B) || c22 || bulk == BULK_14MOM || ctx->df.include_diffusion;
     const bool by_S = (mu_used & MU_S) || c22, by_Q = (mu_used & MU_Q) || c22;
@@ -1100,7 +1109,7 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     const int64_t target = static_cast<int64_t>(ctx->num_cu) * (by_y ? 80 : 160);
     int64_t nch = std::max<int64_t>(1, std::min<int64_t>((target + pw - 1) / pw, milne ? N : (N + 7) / 8));
     int64_t cpc = (N + nch - 1) / nch;
-    if (by_y) cpc = (cpc + kYCells - 1) / kYCells * kYCells;
+    if (by_y && cpc > kYCells) cpc = (cpc + kYCells - 1) / kYCells * kYCells;
     nch = (N + cpc - 1) / cpc;
     // the chunk sums are added in slices of chunks, then the slices
     const int64_t oblk = (nout + 63) / 64;
