@@ -588,7 +588,7 @@ DeltafDev deltaf_dev(iss_ctx* ctx) {
 
 // per-cell coefficients and words of the resident surface; returns when they
 // are ready
-int cell_prep(iss_ctx* ctx) {
+int cell_prep_launch(iss_ctx* ctx) {
     if (ctx->Nneg > 0) {
         HIPCHK(ctx->d_coef_neg.ensure(kCoefRows * ctx->Nneg));
         k_cell_prep<<<(ctx->Nneg + 255) / 256, 256, 0, ctx->stream>>>(ctx->d_cells_neg.p, ctx->Nneg, deltaf_dev(ctx),
@@ -604,8 +604,16 @@ int cell_prep(iss_ctx* ctx) {
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    ctx->tcell_ready = false;
     return ISS_OK;
+}
+
+// (a surface whose preparation fails is dropped: its cells and coefficients
+// no longer belong together)
+int cell_prep(iss_ctx* ctx) {
+    ctx->tcell_ready = false;
+    const int rc = cell_prep_launch(ctx);
+    if (rc) ctx->Nc = ctx->Nneg = ctx->S = 0;
+    return rc;
 }
 
 // the trial kernels' cell words, by the first sampling pass of a surface and
@@ -1424,6 +1432,10 @@ int iss_set_deltaf(iss_ctx* ctx, const iss_deltaf_desc* d) {
         HIPCHK(hipMemcpyAsync(ctx->d_neos.p, d->neos, len * 8, hipMemcpyHostToDevice, ctx->stream));
         ctx->neos_de = d->neos[200 * nc] - d->neos[0];
     }
+    // (before anything of the old delta f is replaced: a failure below must not
+    // leave its yields and trial words in use)
+    ctx->yields_valid = false;
+    ctx->tcell_ready = false;
     ctx->df = *d;
     ctx->df.k11_c0 = ctx->df.k11_c1 = ctx->df.k11_c2 = nullptr;
     ctx->df.neos = nullptr;
@@ -1434,7 +1446,6 @@ int iss_set_deltaf(iss_ctx* ctx, const iss_deltaf_desc* d) {
     if (rc) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->tables_ready = true;
-    ctx->yields_valid = false;
     return cell_prep(ctx);
 }
 

@@ -1,0 +1,79 @@
+"""What the host layer does around its kernels, seen through a stand-in for
+the HIP runtime (tests/fake_hip.cpp): no GPU, no kernel runs.  Every test is a
+program of its own, since the stand-in has to be loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes as C, numpy as np
+fake = C.CDLL({so!r}, mode=C.RTLD_GLOBAL)
+for f in ("fake_launched", "fake_copies", "fake_host_allocs", "fake_largest"):
+    getattr(fake, f).restype = C.c_int64
+fake.fake_known.argtypes = [C.c_void_p, C.c_int64, C.c_int]
+import iss_amd
+
+def launched(part):
+    last = C.c_int64()
+    return fake.fake_launched(part.encode(), C.byref(last)), last.value
+
+def context():
+    ctx = iss_amd.Context(0)
+    ctx.set_species(dict(pid=[211, -211, 2212], mass=[0.14, 0.14, 0.938], g=[1, 1, 2], B=[0, 0, 1], S=[0, 0, 0],
+                         Q=[1, -1, 1], sign=[-1, -1, 1]))
+    return ctx
+
+def cells(n):
+    c = np.zeros((n, 28), np.float32)
+    c[:, 8], c[:, 13] = 1.0, 0.15
+    return c
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    so = os.path.join(str(tmp_path_factory.mktemp("fake")), "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-o", so, os.path.join(ROOT, "tests", "fake_hip.cpp")],
+                   check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE.format(so=so) + body], cwd=ROOT, capture_output=True, text=True,
+                           timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+@pytest.mark.parametrize("change", ["ctx.set_surface_lrf(cells(900))", "ctx.set_deltaf(shear=1)"])
+def test_trial_words_are_not_used_after_a_failed_change(program, change):
+    """Whichever allocation, copy or wait fails in a change of surface or delta
+    f, a pass that the caller runs all the same does not take the words (nor
+    the yields) of what was there before."""
+    program(f"""
+for n in range(1, 40):
+    ctx = context()
+    ctx.set_surface_lrf(cells(100))
+    ctx.sample(1)
+    assert launched("k_trial_cells")[0] > 0
+    ctx.sample(1)
+    fake.fake_reset()
+    ctx.sample(1)
+    assert launched("k_trial_cells")[0] == 0 and launched("k_yield_rows")[0] == 0
+    fake.fake_reset()
+    fake.fake_fail(n, 0)
+    try:
+        {change}
+        failed = False
+    except iss_amd.ISSError:
+        failed = True
+    fake.fake_fail(0, 0)
+    ctx.sample(1)
+    assert ctx.num_cells() == 0 or (launched("k_trial_cells")[0] > 0 and launched("k_yield_rows")[0] > 0), n
+    ctx.close()
+    if not failed:
+        break
+assert n > 1
+""")
