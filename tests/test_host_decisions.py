@@ -27,6 +27,17 @@ def context():
                          Q=[1, -1, 1], sign=[-1, -1, 1]))
     return ctx
 
+def read_list(ctx, nbytes, known=0):
+    # sets a list of that size, reads it back: the read-back's blocking copies and pinned allocations
+    words = np.arange(nbytes // 4, dtype=np.int32)
+    ctx.set_hadrons([words.size // 10], words.view(iss_amd.HADRON_DTYPE))
+    got = np.zeros_like(words)
+    fake.fake_known(got.ctypes.data, nbytes, known)
+    fake.fake_reset()
+    assert ctx.lib.iss_get_hadrons(ctx.h, got.ctypes.data_as(C.c_void_p), words.size // 10) == 0
+    assert np.array_equal(got, words)
+    return fake.fake_copies(), fake.fake_host_allocs()
+
 def cells(n):
     c = np.zeros((n, 28), np.float32)
     c[:, 8], c[:, 13] = 1.0, 0.15
@@ -76,4 +87,14 @@ for n in range(1, 40):
     if not failed:
         break
 assert n > 1
+""")
+
+
+def test_lists_for_memory_that_the_runtime_knows_take_its_copy(program):
+    """Page-locked (1) and device (2) destinations: one copy of the runtime,
+    no staging; pageable ones go through the ring."""
+    program("""
+for known in (1, 2):
+    assert read_list(context(), 100 << 20, known) == (1, 0)
+assert read_list(context(), 100 << 20) == (0, 1)
 """)
