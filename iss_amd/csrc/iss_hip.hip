@@ -219,7 +219,10 @@ struct ReadBack {
         hipError_t e = pin.ensure(kSlots * chunk);
         for (auto& x : ev)
             if (e == hipSuccess && !x) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {  // no pinned memory to be had
+            (void)hipGetLastError();
+            return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+        }
         const int64_t nc = static_cast<int64_t>((bytes + chunk - 1) / chunk);
         std::atomic<int> err{hipSuccess}, team{0}, done[kSlots];
         for (auto& d : done) d = 0;

@@ -98,3 +98,15 @@ for known in (1, 2):
     assert read_list(context(), 100 << 20, known) == (1, 0)
 assert read_list(context(), 100 << 20) == (0, 1)
 """)
+
+
+def test_lists_come_back_where_pinned_memory_runs_out(program):
+    """The ring's slots cannot be had: the runtime's copy, now and at the next
+    list, then the ring once they can."""
+    program("""
+ctx = context()
+for _ in range(2):
+    fake.fake_fail(0, 1)
+    assert read_list(ctx, 100 << 20) == (1, 1)
+assert read_list(ctx, 100 << 20) == (0, 1)
+""")
