@@ -184,17 +184,23 @@ static_assert(kLearnRouteAll == ISS_LEARNED_ROUTE_ALL, "routing constant of the 
 // destination (20 GB/s a thread); the last one to finish a slot sends for the
 // chunk that takes its place.  Chunks of 4 MB hide the ~12 us between two
 // transfers; shorter lists take smaller ones, down to 1 MB, because the first
-// use of a slot pays for its pages (0.35 ms per MB).  Up to kSmall that price
-// and the threads' start cost more than they save, and the list takes the
-// runtime's copy.  379 MB: 21.4 ms before, 7.9 ms now; 34 MB: 1.95 -> 0.85 ms.
+// use of a slot pays for its pages (0.2 ms per MB, once per process where the
+// runtime reuses them).  Up to kSmall the threads' start costs more than they
+// save, and the list takes the runtime's copy.  So do a context's lists until
+// they have come to kRepay bytes, since slots of 3 MB (0.75 ms) save 0.1 ms a
+// list of 5 MB and 0.3 of 12, and slots of 6 MB (1.25 ms) 0.75 of 24: a single
+// list of 5 MB took 0.33 ms by the runtime's copy and 1.0 with its slots.
+// 379 MB: 21.4 ms before, 7.9 ms now; 34 MB: 1.95 -> 0.85 ms.
 // A destination that the runtime knows (page-locked, managed or device memory)
 // takes the runtime's direct copy at any size: into page-locked memory 5 MB
 // take 0.10 ms and 379 MB 7.0, through the ring 0.20 and 8.8, and the threads
 // could not write to device memory.
 struct ReadBack {
     static constexpr int kSlots = 3, kThreads = 4;
-    static constexpr size_t kChunkMin = size_t{1} << 20, kChunkMax = size_t{4} << 20, kSmall = size_t{4} << 20;
+    static constexpr size_t kChunkMin = size_t{1} << 20, kChunkMax = size_t{4} << 20, kSmall = size_t{4} << 20,
+                            kRepay = size_t{24} << 20;
     PinBuf pin;
+    size_t unstaged = 0;  // bytes asked for since the slots were last made
     hipEvent_t ev[kSlots] = {};
     ReadBack() = default;
     ReadBack(const ReadBack&) = delete;
@@ -216,6 +222,12 @@ struct ReadBack {
             return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
         size_t chunk = kChunkMin;
         while (chunk < kChunkMax && bytes / chunk > 16) chunk *= 2;
+        if (pin.cap < kSlots * chunk) {
+            unstaged += bytes;
+            if (unstaged >= kRepay) unstaged = 0;
+            else if (pin.cap > 0) chunk = pin.cap / kSlots;
+            else return hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+        }
         hipError_t e = pin.ensure(kSlots * chunk);
         for (auto& x : ev)
             if (e == hipSuccess && !x) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);

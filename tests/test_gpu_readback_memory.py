@@ -1,6 +1,7 @@
-"""The hadron list's read-back into page-locked memory (the runtime's direct
-copy) and at the edges of a larger page-locked buffer, beside pageable memory:
-the same bytes."""
+"""The hadron list's read-back by the kind of memory and by the context's
+earlier lists: page-locked destinations (the runtime's direct copy), also
+inside a larger page-locked buffer, short pageable lists before and after the
+staging slots exist.  The same bytes everywhere."""
 import ctypes
 
 import numpy as np
@@ -27,4 +28,16 @@ def test_pinned_and_pageable_lists_agree(nbytes):
         assert np.array_equal(got[at:at + nbytes], words.view(np.uint8))
         assert not got[:at].any() and not got[at + nbytes:].any()
     assert np.array_equal(ctx.hadrons().view(np.int32), words)
+    ctx.close()
+
+
+@pytest.mark.parametrize("first", [0, 33 * MB // 40 * 40])
+@pytest.mark.parametrize("nbytes", [4 * MB // 40 * 40 + 40, 5 * MB // 40 * 40, 16 * MB // 40 * 40 + 80])
+def test_short_lists_before_and_after_the_slots(first, nbytes):
+    ctx = iss_amd.Context(0)
+    for n in (first, nbytes):
+        words = np.random.default_rng(n).integers(0, 2 ** 31 - 1, n // 4, dtype=np.int32)
+        ctx.set_hadrons([n // 40], words.view(iss_amd.HADRON_DTYPE))
+        for _ in range(7 if n == nbytes else 1):
+            assert np.array_equal(ctx.hadrons().view(np.int32), words)
     ctx.close()

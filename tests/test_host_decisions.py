@@ -110,3 +110,15 @@ for _ in range(2):
     assert read_list(ctx, 100 << 20) == (1, 1)
 assert read_list(ctx, 100 << 20) == (0, 1)
 """)
+
+
+def test_short_lists_take_the_ring_once_they_repay_its_slots(program):
+    """Lists of 6 MB: the runtime's copy until they have come to 24 MB; one of
+    30 MB takes the ring at once, and short ones after it use its slots."""
+    program("""
+ctx = context()
+MB6, MB30 = 6 * (1 << 20) // 40 * 40 + 40, 30 * (1 << 20) // 40 * 40
+assert [read_list(ctx, MB6) for _ in range(5)] == [(1, 0)] * 3 + [(0, 1), (0, 0)]
+ctx = context()
+assert [read_list(ctx, n) for n in (MB30, MB6, MB30)] == [(0, 1), (0, 0), (0, 0)]
+""")
