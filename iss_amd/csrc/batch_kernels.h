@@ -13,9 +13,10 @@
 //                         those of the next round
 //   k_setup, k_trials     the one-surface kernels, reading the round, the
 //                         hadron count and the output base from the device
-// and after the rounds, for all of them at once (a level of the binomial tree
+// and after the rounds, for many of them at once (a level of the binomial tree
 // is a chain of 13-20 us whatever its number of nodes: 15 rounds of 48
-// surfaces 850 us in the rounds, 85 after them),
+// surfaces 850 us in the rounds, 85 after them; as many rounds as kTreeBytes
+// of nodes hold),
 //   k_batch_multi_*       per (round, surface): Multinomial over its events
 // Every size the kernels need lives on the device, so the host captures one
 // round into a hipGraph and replays it for all rounds (no host round trip,
@@ -62,10 +63,10 @@ __global__ void k_batch_counts(BatchDev b, const double* __restrict__ ctot, int6
     counts[c] = static_cast<uint32_t>(min<int64_t>(cnt, 0xFFFFFFFFll));
 }
 
-// per surface: the root of its event tree (its hadrons of the round), the keyed
+// per surface: the root of its event tree (its hadrons of the round, [rounds][S]), the keyed
 // permutation of its block and the output segment of (round, surface)
 __global__ __launch_bounds__(256) void k_batch_roots(BatchDev b, const int64_t* __restrict__ off, int64_t N,
-                                                    uint64_t seed, int64_t* __restrict__ tree,
+                                                    uint64_t seed, int64_t* __restrict__ roots,
                                                     Permutation* __restrict__ perms, int64_t* __restrict__ seg) {
     // (one workgroup: round and base advance once every thread has read them)
     const uint32_t r = b.round[0];
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(256) void k_batch_roots(BatchDev b, const int64_t* 
         const int64_t h0 = off[b.surf_off[k]], h1 = off[b.surf_off[k + 1]];
         const int64_t H = h1 - h0;
         const int64_t at = static_cast<int64_t>(r) * b.S + k;
-        tree[at] = H;
+        roots[at] = H;
         Permutation p;
         p.init(static_cast<uint64_t>(H > 0 ? H : 1),
                seed ^ (0x5851F42D4C957F2Dull * (static_cast<uint64_t>(k) + 1)) ^ (static_cast<uint64_t>(r) << 40));
@@ -91,15 +92,17 @@ __global__ __launch_bounds__(256) void k_batch_roots(BatchDev b, const int64_t* 
     }
 }
 
-// level d of every (round, surface)'s binomial tree: node (r, k, j) covers the
-// events [j n / 2^d, (j + 1) n / 2^d) of surface k's n = n_k(r)
-__global__ void k_batch_multi_level(BatchDev b, int rounds, const int64_t* __restrict__ parent,
+// level d of the binomial trees of (round, surface), rounds r0 .. r0 + rounds:
+// node (r, k, j) covers the events [j n / 2^d, (j + 1) n / 2^d) of surface k's
+// n = n_k(r).  The nodes of a level: [rounds][S][2^d].
+constexpr int64_t kTreeBytes = int64_t{64} << 20;
+__global__ void k_batch_multi_level(BatchDev b, int r0, int rounds, const int64_t* __restrict__ parent,
                                     int64_t* __restrict__ child, int d, uint64_t seed) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t nodes = static_cast<int64_t>(b.S) << d;  // of a round
     if (i >= nodes * rounds) return;
-    const uint32_t r = static_cast<uint32_t>(i / nodes);
-    const int64_t t = i - r * nodes;
+    const uint32_t r = static_cast<uint32_t>(r0 + i / nodes);
+    const int64_t t = i % nodes;
     const int k = static_cast<int>(t >> d);
     const int64_t j = t & ((1ll << d) - 1);
     const int64_t E = round_events(b.events[k], r, b.R);
@@ -117,13 +120,13 @@ __global__ void k_batch_multi_level(BatchDev b, int rounds, const int64_t* __res
 }
 
 // leaves (2^D >= R): event sizes of (round, surface)
-__global__ void k_batch_multi_leaves(BatchDev b, int rounds, const int64_t* __restrict__ leaf, int D,
+__global__ void k_batch_multi_leaves(BatchDev b, int r0, int rounds, const int64_t* __restrict__ leaf, int D,
                                      uint32_t* __restrict__ evcount) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t nodes = static_cast<int64_t>(b.S) << D;
     if (i >= nodes * rounds) return;
-    const uint32_t r = static_cast<uint32_t>(i / nodes);
-    const int64_t t = i - r * nodes;
+    const uint32_t r = static_cast<uint32_t>(r0 + i / nodes);
+    const int64_t t = i % nodes;
     const int k = static_cast<int>(t >> D);
     const int64_t j = t & ((1ll << D) - 1);
     const int64_t E = round_events(b.events[k], r, b.R);

@@ -434,6 +434,7 @@ struct iss_ctx {
     DBuf<int32_t> d_bevents;
     DBuf<uint32_t> d_bround, d_bevcount;
     DBuf<unsigned long long> d_bbase;
+    DBuf<int64_t> d_broots;
     DBuf<Permutation> d_perms;
     DBuf<int64_t> d_seg;
     DBuf<double> d_lam;
@@ -1262,7 +1263,7 @@ int iss_ctx_destroy(iss_ctx* ctx) {
     ctx->d_cells_neg.release(); ctx->d_coef_neg.release(); ctx->d_srec.release(); ctx->d_sgrid.release();
     ctx->d_smilne.release(); ctx->d_spart.release(); ctx->d_sout.release(); ctx->d_sspec.release();
     ctx->d_surf_off.release(); ctx->d_bevents.release(); ctx->d_bround.release(); ctx->d_bevcount.release();
-    ctx->d_bbase.release(); ctx->d_perms.release(); ctx->d_seg.release(); ctx->d_lam.release();
+    ctx->d_bbase.release(); ctx->d_broots.release(); ctx->d_perms.release(); ctx->d_seg.release(); ctx->d_lam.release();
     for (auto& g : ctx->dgen) g->release();
     ctx->dgen.clear();
     ctx->d_dec_int.release(); ctx->d_dec_dbl.release(); ctx->d_qmu.release(); ctx->d_etab.release(); ctx->d_dnq.release();
@@ -2523,8 +2524,13 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     HIPCHK(ctx->d_perms.ensure(S));
     HIPCHK(ctx->d_seg.ensure(2 * static_cast<size_t>(std::max(rounds, 1)) * S));
     HIPCHK(ctx->d_bevcount.ensure(static_cast<size_t>(std::max(rounds, 1)) * S * R));
-    HIPCHK(ctx->d_tree0.ensure((static_cast<size_t>(S) << D) * std::max(rounds, 1)));
-    HIPCHK(ctx->d_tree1.ensure((static_cast<size_t>(S) << D) * std::max(rounds, 1)));
+    // the event trees' roots, and two levels of the rounds taken together
+    const int64_t tree_nodes = static_cast<int64_t>(S) << D;  // of a round
+    const int tree_rounds = static_cast<int>(std::max<int64_t>(
+        1, std::min<int64_t>(rounds, kTreeBytes / (tree_nodes * static_cast<int64_t>(sizeof(int64_t))))));
+    HIPCHK(ctx->d_broots.ensure(static_cast<size_t>(std::max(rounds, 1)) * S));
+    HIPCHK(ctx->d_tree0.ensure(tree_nodes * tree_rounds));
+    HIPCHK(ctx->d_tree1.ensure(tree_nodes * tree_rounds));
     HIPCHK(ctx->d_scan.ensure(std::max<int64_t>(1, (N + kScanTile - 1) / kScanTile) + 1));
     HIPCHK(ctx->d_bround.ensure(2));
     HIPCHK(ctx->d_bbase.ensure(2));
@@ -2610,7 +2616,7 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     auto round = [&]() {
         if (N > 0) k_batch_counts<<<(N + 255) / 256, 256, 0, ctx->stream>>>(b, ctx->d_ctot.p, N, o->seed, ctx->d_counts.p);
         enqueue_scan(ctx, ctx->d_counts.p, N, ctx->d_scan.p, ctx->d_off.p);
-        k_batch_roots<<<1, 256, 0, ctx->stream>>>(b, ctx->d_off.p, N, o->seed, ctx->d_tree0.p, ctx->d_perms.p,
+        k_batch_roots<<<1, 256, 0, ctx->stream>>>(b, ctx->d_off.p, N, o->seed, ctx->d_broots.p, ctx->d_perms.p,
                                                   ctx->d_seg.p);
         // every slot's cell and species from its cell's yield row (the FP64
         // prefix in LDS, as one surface's pass); the learned rounds' pairs
@@ -2670,17 +2676,19 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
             HIPCHK(hipGetLastError());
         }
     }
-    if (rounds > 0) {
-        // the event sizes of every (round, surface)
-        int64_t* cur = ctx->d_tree0.p;
-        int64_t* nxt = ctx->d_tree1.p;
+    // the event sizes of every (round, surface)
+    for (int r0 = 0; r0 < rounds; r0 += tree_rounds) {
+        const int nr = std::min(tree_rounds, rounds - r0);
+        const int64_t* cur = ctx->d_broots.p + static_cast<int64_t>(r0) * S;
+        int64_t* nxt = ctx->d_tree0.p;
         for (int d = 0; d < D; d++) {
-            const int64_t nodes = (static_cast<int64_t>(S) << d) * rounds;
-            k_batch_multi_level<<<(nodes + 255) / 256, 256, 0, ctx->stream>>>(b, rounds, cur, nxt, d, o->seed);
-            std::swap(cur, nxt);
+            const int64_t nodes = (static_cast<int64_t>(S) << d) * nr;
+            k_batch_multi_level<<<(nodes + 255) / 256, 256, 0, ctx->stream>>>(b, r0, nr, cur, nxt, d, o->seed);
+            cur = nxt;
+            nxt = nxt == ctx->d_tree0.p ? ctx->d_tree1.p : ctx->d_tree0.p;
         }
-        k_batch_multi_leaves<<<((static_cast<int64_t>(S) << D) * rounds + 255) / 256, 256, 0, ctx->stream>>>(
-            b, rounds, cur, D, ctx->d_bevcount.p);
+        k_batch_multi_leaves<<<(tree_nodes * nr + 255) / 256, 256, 0, ctx->stream>>>(b, r0, nr, cur, D,
+                                                                                     ctx->d_bevcount.p);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));

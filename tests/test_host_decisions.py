@@ -122,3 +122,22 @@ assert [read_list(ctx, MB6) for _ in range(5)] == [(1, 0)] * 3 + [(0, 1), (0, 0)
 ctx = context()
 assert [read_list(ctx, n) for n in (MB30, MB6, MB30)] == [(0, 1), (0, 0), (0, 0)]
 """)
+
+
+def test_event_trees_of_many_rounds_stay_small(program):
+    """1000 surfaces, 20,000 events of one of them: 1250 rounds of 16 events.
+    The largest buffer is the event sizes themselves (uint32 [rounds][S][R])."""
+    program("""
+ctx = context()
+ctx.set_surfaces_lrf([cells(1)] * 1000)
+events = np.ones(1000, np.int32)
+events[0] = 20000
+fake.fake_reset()
+ctx.sample_batch(events, events_per_round=16)
+assert 0 < fake.fake_largest() <= 4 * 1250 * 1000 * 16
+assert launched("k_batch_multi_leaves")[0] > 1
+ctx.sample_batch(np.full(1000, 16, np.int32), events_per_round=16)
+fake.fake_reset()
+ctx.sample_batch(np.full(1000, 16, np.int32), events_per_round=16)
+assert launched("k_batch_multi_leaves")[0] == 1
+""")
