@@ -6,11 +6,11 @@
 // cells [surf_off[k], surf_off[k+1])), so the yield pass is one launch over
 // all of them.  Sampling runs in rounds: in round r surface k samples
 // n_k(r) = clamp(E_k - r R, 0, R) events.  One round is
-//   k_batch_counts        Poisson(n_k(r) N_c) hadrons per cell
+//   k_batch_counts        Poisson(n_k(r) N_c) hadrons per cell; names its round
+//                         and output base to the kernels after it
 //   scan                  round-local hadron offsets (all surfaces at once)
 //   k_batch_roots         per surface: its hadron block, its permutation; the
-//                         round and output base of the kernels after it, and
-//                         those of the next round
+//                         next round and its output base
 //   k_setup, k_trials     the one-surface kernels, reading the round, the
 //                         hadron count and the output base from the device
 // and after the rounds, for many of them at once (a level of the binomial tree
@@ -51,8 +51,12 @@ __device__ __forceinline__ int round_events(int E, uint32_t r, int R) {
 __global__ void k_batch_counts(BatchDev b, const double* __restrict__ ctot, int64_t N, uint64_t seed,
                                uint32_t* __restrict__ counts) {
     const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const uint32_t r = b.round[0];
+    if (c == 0) {
+        b.round[1] = r;
+        b.out_base[1] = b.out_base[0];
+    }
     if (c >= N) return;
-    const uint32_t r = *b.round;
     const int k = upper_bound(b.surf_off + 1, 0, b.S, c);
     const int n = round_events(b.events[k], r, b.R);
     int64_t cnt = 0;
@@ -63,33 +67,34 @@ __global__ void k_batch_counts(BatchDev b, const double* __restrict__ ctot, int6
     counts[c] = static_cast<uint32_t>(min<int64_t>(cnt, 0xFFFFFFFFll));
 }
 
-// per surface: the root of its event tree (its hadrons of the round, [rounds][S]), the keyed
-// permutation of its block and the output segment of (round, surface)
-__global__ __launch_bounds__(256) void k_batch_roots(BatchDev b, const int64_t* __restrict__ off, int64_t N,
-                                                    uint64_t seed, int64_t* __restrict__ roots,
-                                                    Permutation* __restrict__ perms, int64_t* __restrict__ seg) {
-    // (one workgroup: round and base advance once every thread has read them)
-    const uint32_t r = b.round[0];
-    const unsigned long long out0 = b.out_base[0];
-    __syncthreads();
-    if (threadIdx.x == 0) {
+// per surface: the root of its event tree (its hadrons of the round,
+// [rounds][S]), the keyed permutation of its block and the output segment of
+// (round, surface).  Every workgroup reads the round and base that
+// k_batch_counts named; one thread moves the next ones on, which none reads.
+// (10^5 surfaces of two cells: 5 us a round; 361 by one workgroup for all.)
+constexpr int kRootThreads = 64;
+__global__ __launch_bounds__(kRootThreads) void k_batch_roots(BatchDev b, const int64_t* __restrict__ off, int64_t N,
+                                                              uint64_t seed, int64_t* __restrict__ roots,
+                                                              Permutation* __restrict__ perms,
+                                                              int64_t* __restrict__ seg) {
+    const int k = blockIdx.x * kRootThreads + threadIdx.x;
+    const uint32_t r = b.round[1];
+    const unsigned long long out0 = b.out_base[1];
+    if (k == 0) {
         b.round[0] = r + 1;
-        b.round[1] = r;
         b.out_base[0] = out0 + static_cast<unsigned long long>(off[N]);
-        b.out_base[1] = out0;
     }
-    for (int k = threadIdx.x; k < b.S; k += blockDim.x) {
-        const int64_t h0 = off[b.surf_off[k]], h1 = off[b.surf_off[k + 1]];
-        const int64_t H = h1 - h0;
-        const int64_t at = static_cast<int64_t>(r) * b.S + k;
-        roots[at] = H;
-        Permutation p;
-        p.init(static_cast<uint64_t>(H > 0 ? H : 1),
-               seed ^ (0x5851F42D4C957F2Dull * (static_cast<uint64_t>(k) + 1)) ^ (static_cast<uint64_t>(r) << 40));
-        perms[k] = p;
-        seg[2 * at] = static_cast<int64_t>(out0) + h0;
-        seg[2 * at + 1] = H;
-    }
+    if (k >= b.S) return;
+    const int64_t h0 = off[b.surf_off[k]], h1 = off[b.surf_off[k + 1]];
+    const int64_t H = h1 - h0;
+    const int64_t at = static_cast<int64_t>(r) * b.S + k;
+    roots[at] = H;
+    Permutation p;
+    p.init(static_cast<uint64_t>(H > 0 ? H : 1),
+           seed ^ (0x5851F42D4C957F2Dull * (static_cast<uint64_t>(k) + 1)) ^ (static_cast<uint64_t>(r) << 40));
+    perms[k] = p;
+    seg[2 * at] = static_cast<int64_t>(out0) + h0;
+    seg[2 * at + 1] = H;
 }
 
 // level d of the binomial trees of (round, surface), rounds r0 .. r0 + rounds:
@@ -135,8 +140,11 @@ __global__ void k_batch_multi_leaves(BatchDev b, int r0, int rounds, const int64
         evcount[(static_cast<int64_t>(r) * b.S + k) * b.R + lo] = static_cast<uint32_t>(leaf[i]);
 }
 
-// per-surface sums of the per-cell totals (one block per surface, FP64)
+// per-surface sums of the per-cell totals (one block per surface, FP64): four
+// waves of it, or sixteen where surfaces have many cells (10^5 surfaces of two
+// cells: 65 us with four, 278 with sixteen)
 constexpr int kLambdaThreads = 1024;
+inline int lambda_threads(int64_t N, int S) { return N / S > kLambdaThreads ? kLambdaThreads : 256; }
 __global__ __launch_bounds__(kLambdaThreads) void k_batch_lambda(const int64_t* __restrict__ surf_off,
                                                      const double* __restrict__ ctot, double* __restrict__ lam) {
     __shared__ double ws[kLambdaThreads / kWave];
@@ -148,7 +156,7 @@ __global__ __launch_bounds__(kLambdaThreads) void k_batch_lambda(const int64_t* 
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.;
-        for (int w = 0; w < kLambdaThreads / kWave; w++) t += ws[w];
+        for (int w = 0; w < static_cast<int>(blockDim.x) / kWave; w++) t += ws[w];
         lam[k] = t;
     }
 }

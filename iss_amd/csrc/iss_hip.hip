@@ -2494,7 +2494,7 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
         const int rc = ensure_tcell(ctx);
         if (rc) return rc;
     }
-    k_batch_lambda<<<S, kLambdaThreads, 0, ctx->stream>>>(ctx->d_surf_off.p, ctx->d_ctot.p, ctx->d_lam.p);
+    k_batch_lambda<<<S, lambda_threads(N, S), 0, ctx->stream>>>(ctx->d_surf_off.p, ctx->d_ctot.p, ctx->d_lam.p);
     HIPCHK(hipGetLastError());
     std::vector<double> lam(S);
     HIPCHK(hipMemcpyAsync(lam.data(), ctx->d_lam.p, sizeof(double) * S, hipMemcpyDeviceToHost, ctx->stream));
@@ -2614,10 +2614,11 @@ int iss_sample_batch(iss_ctx* ctx, const iss_batch_opts* o, const int32_t* n_eve
     af.refill_min = ctx->refill_min[0];
     // one round: only kernel launches, every size read on the device
     auto round = [&]() {
-        if (N > 0) k_batch_counts<<<(N + 255) / 256, 256, 0, ctx->stream>>>(b, ctx->d_ctot.p, N, o->seed, ctx->d_counts.p);
+        k_batch_counts<<<std::max<int64_t>(1, (N + 255) / 256), 256, 0, ctx->stream>>>(b, ctx->d_ctot.p, N, o->seed,
+                                                                                      ctx->d_counts.p);
         enqueue_scan(ctx, ctx->d_counts.p, N, ctx->d_scan.p, ctx->d_off.p);
-        k_batch_roots<<<1, 256, 0, ctx->stream>>>(b, ctx->d_off.p, N, o->seed, ctx->d_broots.p, ctx->d_perms.p,
-                                                  ctx->d_seg.p);
+        k_batch_roots<<<(S + kRootThreads - 1) / kRootThreads, kRootThreads, 0, ctx->stream>>>(
+            b, ctx->d_off.p, N, o->seed, ctx->d_broots.p, ctx->d_perms.p, ctx->d_seg.p);
         // every slot's cell and species from its cell's yield row (the FP64
         // prefix in LDS, as one surface's pass); the learned rounds' pairs
         if (N > 0)

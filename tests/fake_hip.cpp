@@ -27,7 +27,11 @@ namespace {
 constexpr int kSuccess = 0, kInvalid = 1, kNoMemory = 2, kUnknown = 999;
 std::mutex mu;
 std::map<const void*, std::string> kernels;
-std::vector<std::pair<std::string, Dim3>> launches;
+struct Launch {
+    std::string name;
+    Dim3 grid, block;
+};
+std::vector<Launch> launches;
 std::map<void*, size_t> live;
 struct Call {
     Dim3 grid, block;
@@ -63,15 +67,16 @@ void fake_reset() {
     launches.clear();
     n_copies = n_host = largest = 0;
 }
-// workgroups of the launches whose kernel name holds `part`, the last one's; -1: none
-int64_t fake_launched(const char* part, int64_t* last) {
+// the launches whose kernel name holds `part`; workgroups and threads of the last
+int64_t fake_launched(const char* part, int64_t* groups, int64_t* threads) {
     std::lock_guard<std::mutex> g(mu);
     int64_t n = 0;
-    *last = -1;
+    *groups = *threads = -1;
     for (auto& l : launches)
-        if (l.first.find(part) != std::string::npos) {
+        if (l.name.find(part) != std::string::npos) {
             n++;
-            *last = int64_t(l.second.x) * l.second.y * l.second.z;
+            *groups = int64_t(l.grid.x) * l.grid.y * l.grid.z;
+            *threads = int64_t(l.block.x) * l.block.y * l.block.z;
         }
     return n;
 }
@@ -114,9 +119,9 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* shared, void** st
     *stream = c.stream;
     return kSuccess;
 }
-int hipLaunchKernel(const void* f, Dim3 grid, Dim3, void**, size_t, void*) {
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void**, size_t, void*) {
     std::lock_guard<std::mutex> g(mu);
-    launches.emplace_back(kernels[f], grid);
+    launches.push_back({kernels[f], grid, block});
     return kSuccess;
 }
 int hipMalloc(void** p, size_t n) { return allocate(p, n, &fail_device); }

@@ -1,5 +1,6 @@
 """Batches of many surfaces and of many rounds: the layout's invariants where
-the event trees are taken some rounds at a time."""
+the event trees are taken some rounds at a time and where the surfaces are
+more than a workgroup."""
 import numpy as np
 import pytest
 
@@ -47,4 +48,17 @@ def test_event_sizes_of_many_rounds():
     place = ev[:, 0, :].sum(axis=0)
     mean = seg[:, 0, 1].sum() / R
     assert np.abs(place - mean).max() < 6 * np.sqrt(mean)
+    ctx.close()
+
+
+@pytest.mark.parametrize("S", [255, 256, 257, 1000, 2049])
+@pytest.mark.parametrize("use_graph", [0, 1])
+def test_many_surfaces(S, use_graph):
+    """Three rounds of surfaces with 1 to 5 events; rounds replayed and rounds
+    launched give the same list."""
+    events = (1 + np.arange(S) % 5).astype(np.int32)
+    ctx, seg, ev = _batch(S, 2, 3.0 * S, events, 2, use_graph=use_graph)
+    h = ctx.hadrons()
+    other = ctx.sample_batch(events, seed=21, events_per_round=2, use_graph=1 - use_graph)
+    assert other == h.size and np.array_equal(ctx.hadrons(), h)
     ctx.close()

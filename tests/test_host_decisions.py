@@ -18,8 +18,10 @@ fake.fake_known.argtypes = [C.c_void_p, C.c_int64, C.c_int]
 import iss_amd
 
 def launched(part):
-    last = C.c_int64()
-    return fake.fake_launched(part.encode(), C.byref(last)), last.value
+    # how often a kernel was launched; workgroups and threads of the last time
+    groups, threads = C.c_int64(), C.c_int64()
+    n = fake.fake_launched(part.encode(), C.byref(groups), C.byref(threads))
+    return n, groups.value, threads.value
 
 def context():
     ctx = iss_amd.Context(0)
@@ -140,4 +142,17 @@ ctx.sample_batch(np.full(1000, 16, np.int32), events_per_round=16)
 fake.fake_reset()
 ctx.sample_batch(np.full(1000, 16, np.int32), events_per_round=16)
 assert launched("k_batch_multi_leaves")[0] == 1
+""")
+
+
+def test_kernels_of_many_surfaces_fit_them(program):
+    """The kernels over surfaces: at most 64 surfaces a workgroup of a round's
+    roots, and no 16-wave workgroups for the sums of a few cells."""
+    program("""
+for S, n_cells, want in ((1, 2, (1, 256)), (64, 2, (1, 256)), (65, 2, (2, 256)), (1000, 2, (16, 256)), (3, 2000, (1, 1024))):
+    ctx = context()
+    ctx.set_surfaces_lrf([cells(n_cells)] * S)
+    ctx.sample_batch(np.full(S, 3, np.int32), events_per_round=2)
+    assert (launched("k_batch_roots")[1], launched("k_batch_lambda")[2]) == want, (S, want)
+    ctx.close()
 """)
