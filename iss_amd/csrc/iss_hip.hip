@@ -1030,13 +1030,21 @@ double mean_loss(iss_ctx* ctx, int nb) {
 }
 
 // mode 1 takes the rapidities of a (pT, phi) point together where its points
-// fill 60 % of the 64-lane sets: 42 instructions a point against 72
-constexpr bool spec_by_rapidity(int64_t npl) { return 5 * npl >= 3 * 64 * ((npl + 63) / 64); }
+// fill 60 % of the 64-lane sets (42 instructions a point against 72) and its
+// waves, of which each walks more points than one of the general kernel, are
+// two per CU (one species, 112 points, 11 rapidities, 300 cells: 76 waves
+// take 9 us longer than the general kernel's 190) or have two rapidities at most
+bool spec_by_rapidity(int64_t npl, int ny, int64_t ns, int64_t N, int num_cu) {
+    if (5 * npl < 3 * 64 * ((npl + 63) / 64)) return false;
+    const int64_t chunks = spec_y_chunks(ny);
+    return (ny + chunks - 1) / chunks <= 2 ||
+           ns * chunks * spec_y_waves(static_cast<int>(npl)) * ((N + kYCells - 1) / kYCells) >= 2 * num_cu;
+}
 
 template <typename R, int DF>
-void launch_spectra(const SpectraArgs& a, dim3 grid, hipStream_t stream) {
+void launch_spectra(const SpectraArgs& a, bool by_y, dim3 grid, hipStream_t stream) {
     if (a.mode == 1) {
-        if (spec_by_rapidity(a.npT * a.nphi)) k_spectra_y<R, DF><<<grid.x * grid.y, 64, 0, stream>>>(a);
+        if (by_y) k_spectra_y<R, DF><<<grid.x * grid.y, 64, 0, stream>>>(a);
         else k_spectra_points<R><<<grid, 64, 0, stream>>>(a);
     } else if constexpr (sizeof(R) == sizeof(float)) {
         k_spectra32<DF><<<grid, 64, 0, stream>>>(a);
@@ -1097,13 +1105,21 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     // the 321 UrQMD species where mu_S = mu_Q = 0; 314 with all potentials).
     // A charge matters where its potential is not zero on every cell, or
     // where it multiplies a bulk or diffusion term.
-    // Without two species of one mass and statistics (one species, or a few
-    // identified ones) none can share, and the surface is not asked: 15 us of a
-    // small call.
-    std::set<std::pair<double, int>> masses;
-    for (int i = 0; i < ns; i++) masses.emplace(ctx->h_sp[species[i]].mass, ctx->h_sp[species[i]].sign);
-    int mu_used = 0;
-    if (static_cast<int64_t>(masses.size()) < ns) {
+    // Asking the surface for its potentials and sorting the species takes 15
+    // to 25 us, some 10^7 evaluations: calls that cannot spare as many (the
+    // species beyond one per mass and statistics) evaluate every species
+    // (20 species on 300 cells, 10 points: 87 us for 104).
+    const double evals = static_cast<double>(N) * static_cast<double>(npl) * ny;  // of a species
+    const auto spares = [&](int64_t n) { return static_cast<double>(n) * evals > 1e7; };
+    bool share = spares(ns - 1);
+    if (share) {
+        std::set<std::pair<double, int>> masses;
+        for (int i = 0; i < ns; i++) masses.emplace(ctx->h_sp[species[i]].mass, ctx->h_sp[species[i]].sign);
+        share = spares(ns - static_cast<int64_t>(masses.size()));
+    }
+    std::vector<int32_t> spec(species, species + ns);  // the species, then each one's evaluated species
+    std::vector<int32_t> reps;
+    if (share) {
         HIPCHK(ctx->h_pin.ensure(PIN_TOT + sizeof(double) * ctx->Ns));
         HIPCHK(ctx->d_mu_used.ensure(1));
         HIPCHK(hipMemsetAsync(ctx->d_mu_used.p, 0, sizeof(int), ctx->stream));
@@ -1113,21 +1129,23 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
         HIPCHK(hipMemcpyAsync(ctx->h_pin.at<int>(PIN_MU), ctx->d_mu_used.p, sizeof(int), hipMemcpyDeviceToHost,
                               ctx->stream));
         HIPCHK(hipStreamSynchronize(ctx->stream));
-        mu_used = *ctx->h_pin.at<int>(PIN_MU);
-    }
-    const bool c22 = bulk == BULK_22MOM;
-    const bool by_B = (mu_used & MU_B) || c22 || bulk == BULK_14MOM || ctx->df.include_diffusion;
-    const bool by_S = (mu_used & MU_S) || c22, by_Q = (mu_used & MU_Q) || c22;
-    std::vector<int32_t> spec(2 * static_cast<size_t>(ns));  // the species, then each one's evaluated species
-    std::vector<int32_t> reps;
-    std::map<std::tuple<double, int, int, int, int>, int32_t> seen;
-    for (int i = 0; i < ns; i++) {
-        const SpeciesHost& h = ctx->h_sp[species[i]];
-        const auto key = std::make_tuple(h.mass, h.sign, by_B ? h.B : 0, by_S ? h.S : 0, by_Q ? h.Q : 0);
-        const auto it = seen.emplace(key, static_cast<int32_t>(reps.size())).first;
-        if (it->second == static_cast<int32_t>(reps.size())) reps.push_back(species[i]);
-        spec[i] = species[i];
-        spec[ns + i] = it->second;
+        const int mu_used = *ctx->h_pin.at<int>(PIN_MU);
+        const bool c22 = bulk == BULK_22MOM;
+        const bool by_B = (mu_used & MU_B) || c22 || bulk == BULK_14MOM || ctx->df.include_diffusion;
+        const bool by_S = (mu_used & MU_S) || c22, by_Q = (mu_used & MU_Q) || c22;
+        std::map<std::tuple<double, int, int, int, int>, int32_t> seen;
+        for (int i = 0; i < ns; i++) {
+            const SpeciesHost& h = ctx->h_sp[species[i]];
+            const auto key = std::make_tuple(h.mass, h.sign, by_B ? h.B : 0, by_S ? h.S : 0, by_Q ? h.Q : 0);
+            const auto it = seen.emplace(key, static_cast<int32_t>(reps.size())).first;
+            if (it->second == static_cast<int32_t>(reps.size())) reps.push_back(species[i]);
+            spec.push_back(it->second);
+        }
+    } else {
+        for (int i = 0; i < ns; i++) {
+            reps.push_back(species[i]);
+            spec.push_back(i);
+        }
     }
     const int64_t nu = static_cast<int64_t>(reps.size()), nout = nu * npts;
     spec.insert(spec.end(), reps.begin(), reps.end());
@@ -1139,7 +1157,7 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     // cell chunks: several rounds of resident waves over all (chunk,
     // point-wave) pairs, so that the last, partly filled round is short
     // (8 to 16 waves of these kernels fit a CU)
-    const bool by_y = o->mode == 1 && spec_by_rapidity(npl);
+    const bool by_y = o->mode == 1 && spec_by_rapidity(npl, ny, nu, N, ctx->num_cu);
     const int64_t waves = by_y ? int64_t(spec_y_chunks(ny)) * spec_y_waves(static_cast<int>(npl)) : wps;
     const int64_t pw = nu * waves;
     const bool milne = o->mode == 0 && sizeof(R) == sizeof(double);
@@ -1184,19 +1202,25 @@ int run_spectra(iss_ctx* ctx, const iss_spectra_opts* o, const int32_t* species,
     // which terms the delta f has (k_spectra_rec leaves the others zero)
     const bool poly_e = ctx->df.include_diffusion || (shear && ctx->neos == 1);
     const bool const_e = bulk == BULK_RTA || bulk == BULK_CE;
-    if (poly_e) launch_spectra<R, SDF_POLY_E>(a, grid, ctx->stream);
-    else if (const_e) launch_spectra<R, SDF_CONST_E>(a, grid, ctx->stream);
-    else if (shear || bulk != BULK_NONE) launch_spectra<R, SDF_POLY>(a, grid, ctx->stream);
-    else launch_spectra<R, SDF_NONE>(a, grid, ctx->stream);
+    if (poly_e) launch_spectra<R, SDF_POLY_E>(a, by_y, grid, ctx->stream);
+    else if (const_e) launch_spectra<R, SDF_CONST_E>(a, by_y, grid, ctx->stream);
+    else if (shear || bulk != BULK_NONE) launch_spectra<R, SDF_POLY>(a, by_y, grid, ctx->stream);
+    else launch_spectra<R, SDF_NONE>(a, by_y, grid, ctx->stream);
     HIPCHK(hipGetLastError());
     double* sums = ctx->d_spart.p + nch * nout;
     double* slices = sums + nout;
+    // (the last sums are the output where no species shares)
+    const bool shared = nu < ns;
+    const int32_t* scale = shared ? nullptr : ctx->d_sspec.p;
+    double* last = shared ? sums : ctx->d_sout.p;
     k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), static_cast<unsigned>(nsl)), 256, 0, ctx->stream>>>(
-        ctx->d_spart.p, nch, per, nout, nsl > 1 ? slices : sums);
+        ctx->d_spart.p, nch, per, nout, nsl > 1 ? nullptr : scale, a.sp.g, npts, nsl > 1 ? slices : last);
     if (nsl > 1)
-        k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), 1), 256, 0, ctx->stream>>>(slices, nsl, nsl, nout, sums);
-    k_spectra_spread<<<(nall + 255) / 256, 256, 0, ctx->stream>>>(sums, ctx->d_sspec.p, ctx->d_sspec.p + ns, a.sp.g,
-                                                                  npts, nall, ctx->d_sout.p);
+        k_spectra_reduce<<<dim3(static_cast<unsigned>(oblk), 1), 256, 0, ctx->stream>>>(slices, nsl, nsl, nout, scale,
+                                                                                        a.sp.g, npts, last);
+    if (shared)
+        k_spectra_spread<<<(nall + 255) / 256, 256, 0, ctx->stream>>>(sums, ctx->d_sspec.p, ctx->d_sspec.p + ns,
+                                                                      a.sp.g, npts, nall, ctx->d_sout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
     HIPCHK(hipMemcpyAsync(out, ctx->d_sout.p, sizeof(double) * nall, hipMemcpyDeviceToHost, ctx->stream));

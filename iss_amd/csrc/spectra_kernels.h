@@ -740,13 +740,22 @@ __global__ __launch_bounds__(64) void k_spectra64(SpectraArgs a) {
     }
 }
 
+// g / (2 pi hbar c)^3
+__device__ __forceinline__ double spectra_pref(int g) {
+    return static_cast<double>(g) / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
+}
+
 // out[slice][i] = the sum over the slice's chunks (blockIdx.y, `per` chunks
 // each), in a fixed order: 64 consecutive outputs per workgroup, its four
 // waves take every fourth chunk.  Two launches (slices, then the slices'
 // sums) keep the whole chip loading where one thread per output would walk
 // all chunks alone (911 chunks x 2160 outputs: 221 us, now 2 x 9 us for 4546 chunks).
+// species (npts outputs each): the last sums of species that share none, times
+// their prefactors (k_spectra_spread without a launch of its own); null: plain sums.
 __global__ __launch_bounds__(256) void k_spectra_reduce(const double* __restrict__ partial, int64_t nchunks,
-                                                        int64_t per, int64_t n, double* __restrict__ out) {
+                                                        int64_t per, int64_t n, const int32_t* __restrict__ species,
+                                                        const int* __restrict__ g, int64_t npts,
+                                                        double* __restrict__ out) {
     __shared__ double s_sum[4][64];
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
     const int64_t i = static_cast<int64_t>(blockIdx.x) * 64 + lane;
@@ -758,7 +767,10 @@ __global__ __launch_bounds__(256) void k_spectra_reduce(const double* __restrict
     }
     s_sum[w][lane] = s;
     __syncthreads();
-    if (w == 0 && i < n) out[blockIdx.y * n + i] = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
+    if (w == 0 && i < n) {
+        const double v = (s_sum[0][lane] + s_sum[1][lane]) + (s_sum[2][lane] + s_sum[3][lane]);
+        out[blockIdx.y * n + i] = species ? v * spectra_pref(g[species[i / npts]]) : v;
+    }
 }
 
 // out[s] = g_s / (2 pi hbar c)^3 times the sum of the species it shares its
@@ -769,8 +781,7 @@ __global__ void k_spectra_spread(const double* __restrict__ sum, const int32_t* 
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int64_t s = i / npts;
-    const double pref = static_cast<double>(g[species[s]]) / (8. * kPi * kPi * kPi) / (kHbarC * kHbarC * kHbarC);
-    out[i] = sum[pick[s] * npts + (i - s * npts)] * pref;
+    out[i] = sum[pick[s] * npts + (i - s * npts)] * spectra_pref(g[species[s]]);
 }
 
 }  // namespace issdev

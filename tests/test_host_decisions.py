@@ -156,3 +156,28 @@ for S, n_cells, want in ((1, 2, (1, 256)), (64, 2, (1, 256)), (65, 2, (2, 256)),
     assert (launched("k_batch_roots")[1], launched("k_batch_lambda")[2]) == want, (S, want)
     ctx.close()
 """)
+
+
+def test_small_spectra_launch_only_what_they_repay(program):
+    """Species that could share an integrand: the surface is asked for its
+    potentials, and the shared sums spread, only where that spares evaluations
+    worth the question.  Few waves: the general kernel of the rapidities."""
+    program("""
+def spectra(n_cells, idx, n_pT, n_phi, n_y, mode=1):
+    ctx = context()
+    ctx.set_surface_lrf(cells(n_cells))
+    fake.fake_reset()
+    ctx.spectra(idx, np.linspace(0.1, 2.0, n_pT), np.linspace(0, 6.0, n_phi), np.linspace(-2, 2, n_y), np.ones(n_y),
+                mode=mode, precision=64)
+    ctx.close()
+    return [launched(k)[0] for k in ("k_mu_used", "k_spectra_spread", "k_spectra_points", "k_spectra_y")]
+
+for mode, kernel in ((0, [0, 0]), (1, [1, 0])):
+    assert spectra(300, [0, 1, 2], 1, 10, 1, mode) == [0, 0] + kernel
+assert spectra(20000, [0, 2], 15, 48, 11) == [0, 0, 0, 1]       # (two masses)
+assert spectra(20000, [0, 1, 2], 15, 48, 11) == [1, 1, 0, 1]
+assert spectra(300, [0], 7, 16, 11) == [0, 0, 1, 0]
+assert spectra(300, [0], 7, 16, 2) == [0, 0, 0, 1]
+assert spectra(2040, [0], 7, 16, 11) == [0, 0, 1, 0]            # (510 waves)
+assert spectra(2048, [0], 7, 16, 11) == [0, 0, 0, 1]
+""")
