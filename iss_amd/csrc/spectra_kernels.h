@@ -511,12 +511,11 @@ __global__ __launch_bounds__(64) void k_spectra_y(SpectraArgs a) {
 //     instructions per node and wave when every lane forms them).
 //   * 1 / E enters only where the delta f has it (Chapman-Enskog shear, the
 //     relaxation-time and Chapman-Enskog bulk, diffusion): DF.
-//   * exp2 is an 11-term polynomial on [-1/2, 1/2] (relative error 2e-17, 2e-16
-//     with its rounding) and an exponent shift, the reciprocal of the
-//     occupancy a hardware estimate with one third-order step (1 ulp).
+//   * exp2 is a polynomial of degree 11 on [-1/2, 1/2] (relative error 2e-17, 2e-16
+//     with its rounding) and an exponent shift, the occupancy a hardware
+//     reciprocal with one third-order step (1 ulp).
 // Measured at 200,000 cells x 3 species x 720 points x 81 nodes: 98.8 ms
-// with the rest-frame form, 40.5 ms with this kernel (8.6e11 points/s,
-// 31 of the 39 TFMA/s of the FP64 vector unit).
+// with the rest-frame form, 38.8 ms with this kernel (9.0e11 points/s).
 constexpr int kMilneRec = 48;
 enum MilneSlot {
     ML_IT = 0, ML_MB, ML_MS, ML_MQ,    // log2(e) / T and log2(e) mu / T
@@ -558,8 +557,8 @@ __global__ void k_spectra_milne(const double* __restrict__ rec, int64_t N, doubl
                             {1. + u1 * kx, u2 * kx, u3 * kx},
                             {u1 * ky, 1. + u2 * ky, u3 * ky}};
     const double e[4] = {r[ML_E1], r[ML_E2], -u1, -u2};
-    // a temperature or chemical potential that is not a number makes every
-    // point so (the clamped exponent below would drop it)
+    // a temperature or chemical potential that is not a number, or not finite,
+    // makes every point so
     const double poison = 0. * (v[RS_IT] + v[RS_MB] + v[RS_MS] + v[RS_MQ]);
     for (int a = 0; a < 4; a++) {
         r[ML_D1 + a] = e[a] * v[RS_D0] + b[a][0] * v[RS_D1] + b[a][1] * v[RS_D2] + b[a][2] * v[RS_D3] + poison;
@@ -588,14 +587,13 @@ __global__ void k_spectra_milne(const double* __restrict__ rec, int64_t N, doubl
     for (int k = 0; k < kMilneRec; k++) out[i * kMilneRec + k] = r[k];
 }
 
-// 2^x for |x| <= 1000: x = n + f, f in [-1/2, 1/2] (adding 1.5 2^52 rounds to
-// the nearest integer, whose low word is n), 2^f by a polynomial fitted at
-// the Chebyshev nodes of the interval
+// 2^x for every finite x, 0 and infinity beyond the double range: x = n + f, f
+// in [-1/2, 1/2] (n saturates at the ends of the integers), 2^f by a polynomial
+// fitted at the Chebyshev nodes of the interval
 __device__ __forceinline__ double exp2_poly(double x) {
-    const double magic = 6755399441055744.0;
-    const double t = x + magic;
-    const double f = x - (t - magic);
-    const int n = static_cast<int>(__builtin_bit_cast(uint64_t, t));
+    const double t = __builtin_rint(x);
+    const double f = x - t;
+    const int n = static_cast<int>(t);
     double p = 4.455446116749247e-10;
     p = fma(p, f, 7.072590211349959e-09);
     p = fma(p, f, 1.0178059415329878e-07);
@@ -612,10 +610,17 @@ __device__ __forceinline__ double exp2_poly(double x) {
 }
 
 // 1 / d for finite normal d: the hardware estimate (about 2^-24) and one
-// third-order step, within 1 ulp
+// third-order step, within 1 ulp.  occupancy: 0 for d = infinity as well, whose
+// step is not a number and becomes 1.
 __device__ __forceinline__ double rcp_step(double d) {
     const double r = __builtin_amdgcn_rcp(d);
     const double e = fma(-d, r, 1.);
+    return fma(r, fma(e, e, e), r);
+}
+
+__device__ __forceinline__ double occupancy(double d) {
+    const double r = __builtin_amdgcn_rcp(d);
+    const double e = fmin(fma(-d, r, 1.), 1.);
     return fma(r, fma(e, e, e), r);
 }
 
@@ -710,9 +715,7 @@ __global__ __launch_bounds__(64) void k_spectra64(SpectraArgs a) {
                     } else {
                         x = fma(mT[q], nd[0], X0[q]);
                     }
-                    // (2^+-1000: the occupancy is 0, or 1 / sg, to every digit)
-                    x = fmin(fmax(x, -1000.), 1000.);
-                    const double f0 = rcp_step(exp2_poly(x) + sg);
+                    const double f0 = occupancy(exp2_poly(x) + sg);
                     double r = f0 * fma(mT[q], nd[1], Pds[q]);
                     if (DF != SDF_NONE) {
                         double G = fma(mT[q], fma(mT[q], nd[3], fma(px[q], nd[4], fma(py[q], nd[5], nd[6]))), G0[q]);
