@@ -1213,9 +1213,15 @@ __global__ __launch_bounds__(kRowThreads) void k_yield_rows(
             double mu[3];
             row_cell_d<MODE>(a, c, valid, pd, mu);
             const double xb = pd.beta * mu[0], xs = pd.beta * mu[1], xq = pd.beta * mu[2];
-            for (int q = -1; q <= 1; q++) fug[fug_row_d(0, q) * kT] = exp(q * xb);
-            for (int q = -3; q <= 3; q++) fug[fug_row_d(1, q) * kT] = exp(q * xs);
-            for (int q = -2; q <= 2; q++) fug[fug_row_d(2, q) * kT] = exp(q * xq);
+            // (a potential that is not a number leaves no species of the cell
+            // a yield, as in the general series: 0 x it in the row of charge 0)
+            fug[0] = 1. + 0. * (xb + xs + xq);
+            for (int q = -1; q <= 1; q++)
+                if (q) fug[fug_row_d(0, q) * kT] = exp(q * xb);
+            for (int q = -3; q <= 3; q++)
+                if (q) fug[fug_row_d(1, q) * kT] = exp(q * xs);
+            for (int q = -2; q <= 2; q++)
+                if (q) fug[fug_row_d(2, q) * kT] = exp(q * xq);
             const double* dnq_row = (a.dnq && valid) ? a.dnq + c * Ns : nullptr;
             const double* kt = reinterpret_cast<const double*>(s_k);
             const char* fcol = reinterpret_cast<const char*>(fug);
