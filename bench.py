@@ -120,15 +120,27 @@ def cpu_baseline(cells, seconds_target=10.0, total_cells=None):
                               "sample": f"{nev} events, {n1} hadrons in {dt1:.1f} s"}}
 
 
-def traffic_from_profiles(kernel: str):
-    """HBM bytes per launch of `kernel` from the committed rocprofv3 --pmc
-    summary (FETCH_SIZE and WRITE_SIZE, calibrated), or None."""
-    f = os.path.join(ROOT, "profiles", "traffic.json")
+def profile_entry(summary: str, kernel: str, precision: int = 0):
+    """The entry of `kernel` in a committed profile summary, or None.  Of a
+    template's instances: those of the precision (32 or 64) where one is given
+    and profiled, and of these the one with the most dispatches."""
     try:
-        with open(f) as fh:
-            return json.load(fh).get(kernel)
+        with open(os.path.join(ROOT, "profiles", summary)) as fh:
+            u = json.load(fh)
     except (OSError, ValueError):
         return None
+    inst = {k: v for k, v in u.items() if isinstance(v, dict) and k.split("<")[0] == kernel and "<" in k}
+    if not inst:
+        return u.get(kernel)
+    typ = {32: "<float", 64: "<double"}.get(precision, "<")
+    of_type = [v for k, v in inst.items() if typ in k]
+    return max(of_type or inst.values(), key=lambda v: v["dispatches"])
+
+
+def traffic_from_profiles(kernel: str, precision: int = 0):
+    """HBM bytes per launch of `kernel` from the committed rocprofv3 --pmc
+    summary (FETCH_SIZE and WRITE_SIZE, calibrated), or None."""
+    return profile_entry("traffic.json", kernel, precision)
 
 
 def calibration_copy(nbytes):
@@ -181,19 +193,11 @@ def run_steps(ctx, args, proposal, first_event):
     return acc
 
 
-def hw_from_profiles(kernel: str):
+def hw_from_profiles(kernel: str, precision: int = 0):
     """Measured utilisation of `kernel` (VALU issue-slot share, FP32 and BF16
     MFMA FLOP/s against peak) from the committed rocprofv3 counter summary,
     or None."""
-    try:
-        with open(os.path.join(ROOT, "profiles", "utilisation.json")) as fh:
-            u = json.load(fh)
-    except (OSError, ValueError):
-        return None
-    for k, v in u.items():
-        if isinstance(v, dict) and k.split("<")[0] == kernel:
-            return v
-    return None
+    return profile_entry("utilisation.json", kernel, precision)
 
 
 def roofline_valu(kernel, ops, ms):
@@ -228,7 +232,7 @@ def spectra_extra(ctx, sp, n_cells):
         peak = FP32_PEAK_TFLOPS if prec == 32 else FP64_PEAK_TFLOPS
         out[f"fp{prec}"] = {"ms": t, "points_per_s": points / (t * 1e-3),
                             "roofline": {"bound": "valu", "achieved": tf, "peak": peak, "unit": "TFLOP/s",
-                                         "frac": tf / peak, "kernel": "k_spectra"}}
+                                         "frac": tf / peak, "kernel": f"k_spectra{prec}"}}
     return out
 
 
@@ -427,8 +431,9 @@ def main():
     ybytes = yield_bytes(nc, ns, 4 if args.precision == 32 else 8)
     y_gbs = ybytes / (learned["ms_yield"] * 1e-3) / 1e9
     roof_y = {"bound": "hbm", "achieved": y_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-              "frac": y_gbs / HBM_PEAK_GBS, "traffic": traffic_from_profiles("k_yield_rows"), "kernel": "k_yield_rows",
-              "ms": learned["ms_yield"], "bytes": ybytes, "hardware": hw_from_profiles("k_yield_rows")}
+              "frac": y_gbs / HBM_PEAK_GBS, "traffic": traffic_from_profiles("k_yield_rows", args.precision),
+              "kernel": "k_yield_rows", "ms": learned["ms_yield"], "bytes": ybytes,
+              "hardware": hw_from_profiles("k_yield_rows", args.precision)}
     pairs = learned["pairs"] / args.steps
     routed = learned["routed"] / args.steps
     # every pair routed (the autotuner's choice where no pair pays): the
