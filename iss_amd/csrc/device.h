@@ -316,7 +316,6 @@ __device__ __forceinline__ double wave_last(double v) {
     const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(x >> 32), 63);
     return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
-// the sum over all lanes, returned uniformly (from lane 63 of the scan)
 // a 64-bit value of one lane (wave-uniform index), returned uniformly
 template <typename T>
 __device__ __forceinline__ T readlane64(T v, int l) {
@@ -326,6 +325,7 @@ __device__ __forceinline__ T readlane64(T v, int l) {
     const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(x >> 32), l);
     return __builtin_bit_cast(T, (static_cast<uint64_t>(hi) << 32) | lo);
 }
+// the sum over all lanes, returned uniformly (from lane 63 of the scan)
 __device__ __forceinline__ double wave_sum_dpp(double v) { return wave_last(wave_scan_dpp(v)); }
 // Running maximum over the lanes up to this one, in the steps of
 // wave_scan_dpp; for non-negative values (lanes without a source take 0)
@@ -394,18 +394,6 @@ __device__ __forceinline__ T wave_inclusive_scan(T v) {
     for (int d = 1; d < kWave; d <<= 1) {
         const T o = __shfl_up(v, d, kWave);
         if (lane >= d) v += o;
-    }
-    return v;
-}
-
-// running maximum over the lanes up to this one
-template <typename T>
-__device__ __forceinline__ T wave_inclusive_max(T v) {
-    const int lane = threadIdx.x & (kWave - 1);
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const T o = __shfl_up(v, d, kWave);
-        if (lane >= d) v = v > o ? v : o;
     }
     return v;
 }

@@ -1330,15 +1330,6 @@ int iss_set_species(iss_ctx* ctx, const iss_species_desc* sp) {
         k.sgn = static_cast<float>(sp->sign[i]);
         k.md = sp->mass[i];
         k.prefd = static_cast<double>(sp->degeneracy[i]) * uf;
-        k.m2 = static_cast<float>(sp->mass[i] * sp->mass[i]);
-        k.m3 = static_cast<float>(sp->mass[i] * sp->mass[i] * sp->mass[i]);
-        k.m4 = static_cast<float>(sp->mass[i] * sp->mass[i] * sp->mass[i] * sp->mass[i]);
-        k.g = static_cast<float>(sp->degeneracy[i]);
-        k.Bi = sp->baryon[i];
-        k.Si = sp->strange[i];
-        k.Qi = sp->charge[i];
-        k.pad = 0;
-        k.md20 = 20. * sp->mass[i];
     }
     HIPCHK(ctx->d_mass.ensure(Ns));
     HIPCHK(ctx->d_ints.ensure(6 * Ns));
@@ -1353,9 +1344,9 @@ int iss_set_species(iss_ctx* ctx, const iss_species_desc* sp) {
     HIPCHK(hipMemcpyAsync(ctx->d_tspec.p, tsp.data(), sizeof(TSpec) * Ns, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->Ns = Ns;
-    // the leading species below 0.7 GeV take the 10-term series (the row
-    // pass gives them lanes of their own; lighter species further down the
-    // list, if any, are still summed correctly, by the one-term lanes' loop)
+    // the leading species below 0.7 GeV take the 10-term series (a lighter
+    // species further down the list sends the whole row pass to the general
+    // series)
     ctx->nlight = 0;
     while (ctx->nlight < std::min(Ns, kLightMax) && sp->mass[ctx->nlight] < 0.7) ctx->nlight++;
     ctx->light_beyond = false;

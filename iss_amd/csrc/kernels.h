@@ -42,7 +42,6 @@ constexpr int kMaxSpecies = 512;
 // the species CDF's row stride: rows start on 128-byte boundaries, so that
 // the yield pass stores whole 128-byte lines (16 species per staging chunk)
 __host__ __device__ constexpr int cdf_stride(int ns) { return (ns + 15) & ~15; }
-constexpr int kMaxChunks = kMaxSpecies / kWave;
 constexpr int kPTabLen = 2001;
 
 enum BulkMode { BULK_NONE = 0, BULK_RTA = 1, BULK_14MOM = 11, BULK_22MOM = 20, BULK_CE = 21 };
@@ -62,11 +61,6 @@ struct SpeciesDev {
 struct SpeciesK {
     float m, pref, B, S, Q, sgn;
     double md, prefd;
-    // the one-term yields of the row pass: m^2, m^3, m^4, degeneracy, the
-    // charges as integers, 20 m (FP64: places m / T in the K table)
-    float m2, m3, m4, g;
-    int Bi, Si, Qi, pad;
-    double md20;
 };
 
 // Species constants of the yield-row pass (padded to whole 64-byte segments

@@ -640,21 +640,16 @@ __device__ __forceinline__ float yield_fp64_cold(const YieldArgs& a, int64_t c, 
 struct RowCellF {
     float T, beta, Pi, pdc;
     double betad;
-    float eBp, eBm, eSp, eSm, eQp, eQm;  // e^{+beta mu}, e^{-beta mu} of the three charges
-    float muB, muS, muQ, dsu;
-    float k1, k2, k3, k4, k5;   // per-cell bulk products (MODE-dependent)
+    float k1, k2, k3;   // per-cell bulk products (MODE-dependent)
 };
 
 template <int MODE>
 __device__ __forceinline__ void row_cell_f(const YieldArgs& a, int64_t c, bool valid, RowCellF& p, float cf[6]) {
     const int64_t Nc = a.Nc;
-    double T = 0.15, muB = 0., muS = 0., muQ = 0., dsu = 0., Pi = 0.;
+    double T = 0.15, dsu = 0., Pi = 0.;
     double cd[6] = {0., 0., 0., 0., 0., 0.};
     if (valid) {
         T = a.cells[F_T * Nc + c];
-        muB = a.cells[F_MUB * Nc + c];
-        muS = a.cells[F_MUS * Nc + c];
-        muQ = a.cells[F_MUQ * Nc + c];
         dsu = a.cells[F_DA0 * Nc + c];
         if (MODE != BULK_NONE) {
             Pi = a.cells[F_PI * Nc + c];
@@ -663,10 +658,6 @@ __device__ __forceinline__ void row_cell_f(const YieldArgs& a, int64_t c, bool v
         }
     }
     p.T = static_cast<float>(T);
-    p.muB = static_cast<float>(muB);
-    p.muS = static_cast<float>(muS);
-    p.muQ = static_cast<float>(muQ);
-    p.dsu = static_cast<float>(dsu);
     p.betad = 1. / T;
     p.beta = static_cast<float>(p.betad);
     // the general series divides the float Pi by hbar c in FP32 (RTA)
@@ -674,17 +665,10 @@ __device__ __forceinline__ void row_cell_f(const YieldArgs& a, int64_t c, bool v
     if (MODE == BULK_RTA) Pif = Pif / static_cast<float>(kHbarC);
     p.Pi = Pif;
     p.pdc = static_cast<float>(dsu) * static_cast<float>(1.0 / (kHbarC * kHbarC * kHbarC) / (2. * kPi * kPi));
-    const double xb = p.betad * muB, xs = p.betad * muS, xq = p.betad * muQ;
-    p.eBp = static_cast<float>(exp(xb));
-    p.eBm = static_cast<float>(exp(-xb));
-    p.eSp = static_cast<float>(exp(xs));
-    p.eSm = static_cast<float>(exp(-xs));
-    p.eQp = static_cast<float>(exp(xq));
-    p.eQm = static_cast<float>(exp(-xq));
 #pragma unroll
     for (int k = 0; k < 6; k++) cf[k] = static_cast<float>(cd[k]);
     const double T2 = T * T;
-    p.k1 = p.k2 = p.k3 = p.k4 = p.k5 = 0.f;
+    p.k1 = p.k2 = p.k3 = 0.f;
     if (MODE == BULK_14MOM) {
         p.k1 = static_cast<float>(T * cd[0]);        // m^4 T C0 K2
         p.k2 = static_cast<float>(T2 * cd[1]);       // m^2 B T^2 C1 (m b K1 + 3 K2)
@@ -692,12 +676,6 @@ __device__ __forceinline__ void row_cell_f(const YieldArgs& a, int64_t c, bool v
     } else if (MODE == BULK_RTA || MODE == BULK_CE) {
         p.k1 = static_cast<float>(static_cast<double>(cf[0]) * static_cast<double>(cf[1]) * T);  // c0 c1 T m^2 B1
         p.k2 = cf[0];                                                                              // - c0 m^3 / 3 K1
-    } else if (MODE == BULK_22MOM) {
-        p.k1 = static_cast<float>(T * cd[2]);            // m^4 T c2 K2
-        p.k2 = static_cast<float>(T2 * (cd[1] - cd[2])); // m^3 T^2 (c1 - c2) B2
-        p.k3 = static_cast<float>(T2 * cd[3]);           // m^2 T^2 (B c3 + S c4 + Q c5) B1
-        p.k4 = static_cast<float>(T2 * cd[4]);
-        p.k5 = static_cast<float>(T2 * cd[5]);
     }
 }
 
