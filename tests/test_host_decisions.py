@@ -181,3 +181,17 @@ assert spectra(300, [0], 7, 16, 2) == [0, 0, 0, 1]
 assert spectra(2040, [0], 7, 16, 11) == [0, 0, 1, 0]            # (510 waves)
 assert spectra(2048, [0], 7, 16, 11) == [0, 0, 0, 1]
 """)
+
+
+def test_sparse_rounds_take_the_sparse_pick(program):
+    """512 cells a CU and at most two slots a cell; else the general pick."""
+    program("""
+for n_cells, want in ((131071, [0, 1]), (131072, [1, 0])):
+    ctx = context()
+    ctx.set_surfaces_lrf([cells(n_cells)])
+    fake.fake_reset()
+    ctx.sample_batch(np.full(1, 2, np.int32), events_per_round=2, use_graph=1)
+    few, all_picks = launched("k_pick_few")[0], launched("k_pick")[0]
+    assert [few, all_picks - few] == want, (n_cells, few, all_picks)
+    ctx.close()
+""")
