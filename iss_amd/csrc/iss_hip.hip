@@ -184,12 +184,13 @@ static_assert(kLearnRouteAll == ISS_LEARNED_ROUTE_ALL, "routing constant of the 
 // destination (20 GB/s a thread); the last one to finish a slot sends for the
 // chunk that takes its place.  Chunks of 4 MB hide the ~12 us between two
 // transfers; shorter lists take smaller ones, down to 1 MB, because the first
-// use of a slot pays for its pages (0.2 ms per MB, once per process where the
-// runtime reuses them).  Up to kSmall the threads' start costs more than they
-// save, and the list takes the runtime's copy.  So do a context's lists until
-// they have come to kRepay bytes, since slots of 3 MB (0.75 ms) save 0.1 ms a
-// list of 5 MB and 0.3 of 12, and slots of 6 MB (1.25 ms) 0.75 of 24: a single
-// list of 5 MB took 0.33 ms by the runtime's copy and 1.0 with its slots.
+// use of a slot pays for its pages (0.2 ms per MB in a process without free
+// ones).  Up to kSmall the threads' start costs more than they save, and the
+// list takes the runtime's copy.  So do a context's lists until they have come
+// to kRepay bytes: slots of 3 MB (0.75 ms, or 0.1 on pages of an earlier
+// context) save 0.1 ms a list of 5 MB, 0.3 of 12 and 0.4 of 16, so short lists
+// repay them late (a process's single list of 5 MB took 0.33 ms by the
+// runtime's copy and 1.0 with its slots) and lists from 12 MB by the third.
 // 379 MB: 21.4 ms before, 7.9 ms now; 34 MB: 1.95 -> 0.85 ms.
 // A destination that the runtime knows (page-locked, managed or device memory)
 // takes the runtime's direct copy at any size: into page-locked memory 5 MB
@@ -198,7 +199,7 @@ static_assert(kLearnRouteAll == ISS_LEARNED_ROUTE_ALL, "routing constant of the 
 struct ReadBack {
     static constexpr int kSlots = 3, kThreads = 4;
     static constexpr size_t kChunkMin = size_t{1} << 20, kChunkMax = size_t{4} << 20, kSmall = size_t{4} << 20,
-                            kRepay = size_t{24} << 20;
+                            kRepay = size_t{12} << 20;
     PinBuf pin;
     size_t unstaged = 0;  // bytes asked for since the slots were last made
     hipEvent_t ev[kSlots] = {};

@@ -115,14 +115,15 @@ assert read_list(ctx, 100 << 20) == (0, 1)
 
 
 def test_short_lists_take_the_ring_once_they_repay_its_slots(program):
-    """Lists of 6 MB: the runtime's copy until they have come to 24 MB; one of
-    30 MB takes the ring at once, and short ones after it use its slots."""
+    """Lists of 5 MB: the runtime's copy until they have come to 12 MB; one of
+    13 MB takes the ring at once, and short ones after it use its slots."""
     program("""
 ctx = context()
-MB6, MB30 = 6 * (1 << 20) // 40 * 40 + 40, 30 * (1 << 20) // 40 * 40
-assert [read_list(ctx, MB6) for _ in range(5)] == [(1, 0)] * 3 + [(0, 1), (0, 0)]
+MB5, MB13, MB30 = (n * (1 << 20) // 40 * 40 for n in (5, 13, 30))
+assert [read_list(ctx, MB5) for _ in range(4)] == [(1, 0)] * 2 + [(0, 1), (0, 0)]
 ctx = context()
-assert [read_list(ctx, n) for n in (MB30, MB6, MB30)] == [(0, 1), (0, 0), (0, 0)]
+assert [read_list(ctx, n) for n in (MB13, MB5, MB13)] == [(0, 1), (0, 0), (0, 0)]
+assert [read_list(ctx, n) for n in (MB30, MB5, MB30)] == [(0, 1), (0, 0), (0, 0)]
 """)
 
 
